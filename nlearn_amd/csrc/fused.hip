@@ -15,6 +15,8 @@
 // vector per lane), wavefront butterflies for the row statistics, no LDS in
 // the forward. Parameter-gradient sums are per-workgroup partial rows combined
 // in a fixed order by a second kernel (deterministic, no atomics).
+#include <type_traits>
+
 #include "common.h"
 
 namespace nl {
@@ -391,31 +393,40 @@ __global__ __launch_bounds__(128) void embed_fwd_kernel(int S, int D, const int3
 // of a bucket are then contiguous and in increasing t, and the lists hold
 // exactly the valid tokens.
 //
-// embed_bwd_kernel (one wave per workgroup):
+// embed_bwd_kernel:
 // * workgroups [0, S) form dpos[s] (+)= sum_b dx[b, s] in batch order;
-// * workgroup S + g owns the token-table rows [g R, g R + R) (R divides W) in
-//   LDS, walks its bucket's segments in order and adds dx[t] to row ids[t] for the
-//   positions whose id it owns: each (row, column) is summed by one lane in
-//   increasing t (np.add.at's order). Every owned row is then written, zero when
-//   no token has its id, so dtok needs no zeroing first.
-constexpr int kEmbTokLds = 16384;  // bytes of LDS per row workgroup (R = 16384 / (4 D) rows)
+// * workgroup S + g owns R token-table rows of one bucket (their sums in LDS)
+//   and walks the bucket's list 512 entries at a time: its waves sort the
+//   entries of the owned rows by row (ballots keep the tokens of a row in
+//   increasing t), then every thread adds its CW columns of dx[t] along the
+//   sorted entries, holding the current row's sum in registers: each (row,
+//   column) is summed by one thread in increasing t (np.add.at's order). Every
+//   owned row is then written, zero when no token has its id, so dtok needs no
+//   zeroing first.
+//   What bounds it: ids as spread as a uniform draw leave mostly the write of
+//   dtok (103 MB at 50257 x 512), hence few registers and many workgroups per
+//   CU. Ids with the 1/rank frequencies of text put a fifth of all tokens on
+//   the first 8 rows, one serial chain by contract: what counts there is how
+//   many dx rows are in flight and how few instructions an entry takes. The
+//   whole backward at 50257 x 512, against one wave per 8 rows that loads and
+//   adds one token at a time: 8 x 512 tokens of such ids 545 -> 72 us, 32 x 512
+//   2150 -> 245 us; of uniform ids 27 -> 30 and 38 -> 39 us.
+constexpr int kEmbTokLds = 16384;  // a bucket is a whole number of 16384 / (4 D)-row groups
 constexpr int kEmbBuckets = 256;   // target number of buckets
 constexpr int kEmbParts = 4;       // token ranges per bucket (one scanning workgroup each)
-constexpr int kEmbMaxBuckets = 256;  // W = ceil(vocab / 256) rounded up to R: at most 256 buckets
+constexpr int kEmbMaxBuckets = 256;  // W = ceil(vocab / 256) rounded up to a whole group: at most 256 buckets
+constexpr int kEmbChunk = 512;     // list entries sorted into per-row lists at a time
 
 struct EmbPlan {
-  int R;        // token-table rows per row workgroup
-  int W;        // rows per bucket, a multiple of R
+  int W;        // rows per bucket
   int buckets;  // ceil(vocab / W)
-  int64_t groups;
 };
 EmbPlan emb_plan(int D, int vocab) {
   EmbPlan p;
-  p.R = std::max(1, kEmbTokLds / (D * 4));
+  const int unit = std::max(1, kEmbTokLds / (D * 4));
   const int want = (vocab + kEmbBuckets - 1) / kEmbBuckets;
-  p.W = (want + p.R - 1) / p.R * p.R;
+  p.W = (want + unit - 1) / unit * unit;
   p.buckets = (vocab + p.W - 1) / p.W;
-  p.groups = ((int64_t)vocab + p.R - 1) / p.R;
   return p;
 }
 
@@ -507,16 +518,27 @@ __global__ __launch_bounds__(256) void embed_bucket_kernel(int T, int vocab, int
   }
 }
 
-__global__ __launch_bounds__(64) void embed_bwd_kernel(int B, int S, int D, const int32_t* __restrict__ ids,
-                                                       const uint16_t* __restrict__ dx, float* __restrict__ dtok,
-                                                       int vocab, int R, int W, const int* __restrict__ counts,
-                                                       const int* __restrict__ offsets,
-                                                       const int2* __restrict__ lists, float* __restrict__ dpos,
-                                                       int accumulate) {
-  const int lane = threadIdx.x;
+// CW bf16 columns of a dx row (CW / 2 dwords; rows are 8-byte aligned)
+template <int CW>
+struct EmbCols {
+  uint32_t d[CW / 2];
+};
+
+// accumulators per row: a column for every lane of the waves that cover D
+template <int CW>
+__host__ __device__ constexpr int emb_pitch(int D) { return (D + 64 * CW - 1) / (64 * CW) * (64 * CW); }
+
+template <int CW, int R>
+__global__ __launch_bounds__(256, CW == 2 ? 7 : 6) void embed_bwd_kernel(int B, int S, int D, const uint16_t* __restrict__ dx,
+                                                        float* __restrict__ dtok, int vocab, int W, int groups,
+                                                        const int* __restrict__ counts,
+                                                        const int* __restrict__ offsets,
+                                                        const int2* __restrict__ lists, float* __restrict__ dpos,
+                                                        int accumulate) {
+  const int tid = threadIdx.x, nt = blockDim.x;
   if ((int)blockIdx.x < S) {
     const int s = blockIdx.x;
-    for (int c = lane; c < D; c += 64) {
+    for (int c = tid; c < D; c += nt) {
       float a = 0.f;
 #pragma unroll 8
       for (int b = 0; b < B; ++b) a += bf16_to_f32(dx[((int64_t)b * S + s) * D + c]);
@@ -525,45 +547,168 @@ __global__ __launch_bounds__(64) void embed_bwd_kernel(int B, int S, int D, cons
     }
     return;
   }
-  extern __shared__ f32x4 emb_acc4[];
-  float* acc = reinterpret_cast<float*>(emb_acc4);
-  const int T = B * S;
-  const int v0 = ((int)blockIdx.x - S) * R;
-  const int nrows = min(R, vocab - v0);
-  const int n4 = nrows * D / 4;
-  for (int i = lane; i < n4; i += 64) emb_acc4[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  __syncthreads();
-  const int b = v0 / W;
-  // the bucket's segments in order: every position of segment k precedes those of k + 1
-  for (int kp = 0; kp < (T > 0 ? kEmbParts : 0); ++kp) {
-    const int n = counts[b * kEmbParts + kp];
-    const int2* list = lists + offsets[b * kEmbParts + kp];
-    for (int j0 = 0; j0 < n; j0 += 64) {
-      const int2 e = j0 + lane < n ? list[j0 + lane] : int2{0, -1};
-      const int t = e.x, id = e.y;
-      uint64_t hits = __ballot((uint32_t)(id - v0) < (uint32_t)nrows);
-      while (hits) {
-        const int l = __builtin_ctzll(hits);
-        hits &= hits - 1;
-        const int tl = __builtin_amdgcn_readlane(t, l);
-        const int row = __builtin_amdgcn_readlane(id, l) - v0;
-        const uint16_t* src = dx + (int64_t)tl * D;
-        float* dst = acc + row * D;
-        for (int c = lane * 4; c < D; c += 256) {
-          const u32x2 x = *reinterpret_cast<const u32x2*>(src + c);
-          f32x4 a = *reinterpret_cast<const f32x4*>(dst + c);
-          a[0] += bf16_lo(x[0]);
-          a[1] += bf16_hi(x[0]);
-          a[2] += bf16_lo(x[1]);
-          a[3] += bf16_hi(x[1]);
-          *reinterpret_cast<f32x4*>(dst + c) = a;
-        }
+  typedef __attribute__((__vector_size__(CW * sizeof(float)))) float facc;
+  __shared__ int2 sorted[kEmbChunk];              // (t, row) of the chunk's owned entries, by row, then t
+  extern __shared__ __attribute__((aligned(16))) float acc[];  // [R][pitch]; a thread touches its own columns only
+  const int lane = tid & 63, nw = nt >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = (int)blockIdx.x - S;
+  const int b = g / groups;
+  const int64_t v0 = (int64_t)b * W + (int64_t)(g - b * groups) * R;
+  const int64_t vend = min((int64_t)vocab, (int64_t)(b + 1) * W);
+  if (v0 >= vend) return;
+  const int nrows = (int)min((int64_t)R, vend - v0);
+
+  // the segments of a bucket are contiguous: one list of n entries
+  int n = 0;
+  const int2* list = lists;
+  if (B > 0 && S > 0) {
+#pragma unroll
+    for (int k = 0; k < kEmbParts; ++k) n += counts[b * kEmbParts + k];
+    list += offsets[b * kEmbParts];
+  }
+  constexpr int PER = kEmbChunk / 64;
+  int et[PER], er[PER];  // the chunk's entries: token, row - v0 (negative or >= R: another workgroup's)
+  auto fetch = [&](int c0) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int2 e = c0 + i * 64 + lane < n ? list[c0 + i * 64 + lane] : int2{0, -1};
+      et[i] = e.x;
+      er[i] = e.y - (int)v0;
+    }
+  };
+  const int pitch = emb_pitch<CW>(D);
+  uint32_t seen = 0;  // rows with an accumulator
+  if (n > 0) fetch(0);
+  for (int c0 = 0; c0 < n; c0 += kEmbChunk) {
+    // every wave counts the chunk's entries of each owned row; wave r % nw then
+    // writes row r's, in order, behind those of the rows before it
+    uint32_t has = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (__ballot((uint32_t)er[i] < (uint32_t)R)) has |= 1u << i;
+    int m = 0;
+    uint32_t now = 0;  // rows with tokens in this chunk
+    if (has) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        int cur = m;
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+          if (has >> i & 1) {
+            const bool hit = er[i] == r;
+            const uint64_t k = __ballot(hit);
+            if (hit && r % nw == wave)
+              sorted[cur + __builtin_amdgcn_mbcnt_hi((uint32_t)(k >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)k, 0))] =
+                  int2{et[i], r};
+            cur += __popcll(k);
+          }
+        if (cur > m) now |= 1u << r;
+        m = cur;
       }
     }
+    if (c0 + kEmbChunk < n) fetch(c0 + kEmbChunk);
+    if (m == 0) continue;  // the same in every wave
+    __syncthreads();
+    constexpr int DEPTH = CW == 2 ? 32 : 16, REST = 8;
+    // a wave's lanes past column D read the row's last columns and sum them into
+    // accumulators of their own, which nobody stores: no lane masks in the loop
+    for (int w0 = wave * 64 * CW; w0 < D; w0 += nt * CW) {
+      const int c = w0 + lane * CW;
+      const int co = min(c, D - CW);
+      float* ac = acc + c;
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if ((now & ~seen) >> r & 1) *reinterpret_cast<facc*>(ac + r * pitch) = facc{};
+      int row = __builtin_amdgcn_readfirstlane(sorted[0].y);  // the row whose sum is in `cur`
+      facc cur = *reinterpret_cast<const facc*>(ac + row * pitch);
+      auto add = [&](const EmbCols<CW>& x) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < CW / 2; ++e) {
+          cur[2 * e] += bf16_lo(x.d[e]);
+          cur[2 * e + 1] += bf16_hi(x.d[e]);
+        }
+      };
+      // entries i .. i + N - 1 (those past m repeat the last and are not added):
+      // every lane forms one entry's row address, so a load costs two lane reads
+      auto batch = [&](auto nn, int i) __attribute__((always_inline)) {
+        constexpr int N = decltype(nn)::value;
+        const int k = min(i + (lane & (N - 1)), m - 1);
+        const int2 e = sorted[k];
+        const uint64_t ad = (uint64_t)(dx + (int64_t)e.x * D);
+        const bool end = i + (lane & (N - 1)) >= m;
+        const uint32_t stop = (uint32_t)__ballot(end || (k > 0 && sorted[k - 1].y != e.y));  // not simply "add to cur"
+        EmbCols<CW> x[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)ad, j);
+          const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(ad >> 32), j);
+          const uint16_t* q = reinterpret_cast<const uint16_t*>(((uint64_t)hi << 32) | lo) + (uint32_t)co;
+          if constexpr (CW == 2) x[j].d[0] = *reinterpret_cast<const uint32_t*>(q);
+          else {
+            const u32x2 v = *reinterpret_cast<const u32x2*>(q);
+            x[j].d[0] = v[0];
+            x[j].d[1] = v[1];
+          }
+        }
+#pragma unroll
+        for (int j0 = 0; j0 < N; j0 += 4) {
+          if ((stop >> j0 & 15u) == 0) {
+#pragma unroll
+            for (int j = j0; j < j0 + 4; ++j) add(x[j]);
+          } else {
+#pragma unroll
+            for (int j = j0; j < j0 + 4; ++j) {
+              if (i + j >= m) continue;
+              const int r = __builtin_amdgcn_readlane(e.y, j);
+              if (r != row) {
+                *reinterpret_cast<facc*>(ac + row * pitch) = cur;
+                cur = *reinterpret_cast<const facc*>(ac + r * pitch);
+                row = r;
+              }
+              add(x[j]);
+            }
+          }
+        }
+      };
+      for (int i = 0; i < m;) {
+        if (m - i > REST) {
+          batch(std::integral_constant<int, DEPTH>{}, i);
+          i += DEPTH;
+        } else {
+          batch(std::integral_constant<int, REST>{}, i);
+          i += REST;
+        }
+      }
+      *reinterpret_cast<facc*>(ac + row * pitch) = cur;
+    }
+    seen |= now;
+    __syncthreads();  // the sorted entries are rewritten by the next chunk
   }
-  __syncthreads();
-  f32x4* out = reinterpret_cast<f32x4*>(dtok + (int64_t)v0 * D);
-  for (int i = lane; i < n4; i += 64) out[i] = emb_acc4[i];
+  // the owned rows are contiguous in dtok: 16 bytes per lane (the last barrier
+  // made every column's sum visible)
+  const int d4 = D / 4, n4 = nrows * d4;
+  f32x4* out = reinterpret_cast<f32x4*>(dtok + v0 * D);
+  if (seen == 0) {
+    for (int i = tid; i < n4; i += nt) out[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    return;
+  }
+  for (int i = tid; i < n4; i += nt) {
+    const int r = i / d4;
+    out[i] = seen >> r & 1 ? *reinterpret_cast<const f32x4*>(acc + r * pitch + (i - r * d4) * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+}
+
+// rows per row workgroup: at most 16 KB of accumulators
+int emb_rows(int D) { return D <= 512 ? 8 : D <= 1024 ? 4 : D <= 2048 ? 2 : 1; }
+
+template <int CW, int R>
+void launch_embed_bwd(hipStream_t st, int64_t grid, int batch, int seq, int D, const uint16_t* dx, float* dtok,
+                      int vocab, int W, const int* counts, const int* offsets, const int2* lists, float* dpos,
+                      int accumulate) {
+  const int nt = std::min(256, (D / CW + 63) / 64 * 64);
+  hipLaunchKernelGGL((embed_bwd_kernel<CW, R>), dim3((unsigned)grid), dim3(nt), R * emb_pitch<CW>(D) * sizeof(float), st, batch, seq,
+                     D, dx, dtok, vocab, W, (W + R - 1) / R, counts, offsets, lists, dpos, accumulate);
 }
 
 int vectors_per_lane(int D) {
@@ -785,7 +930,8 @@ extern "C" int nl_embedding_bwd(void* stream, int batch, int seq, int D, int voc
     return nl_set_error(NL_EALIGN, "embedding_bwd: dtok must be 16-byte and dx 8-byte aligned");
   if (T64 > 0x7fffffff - 1024) return nl_set_error(NL_EINVAL, "embedding_bwd: too many tokens");
   const EmbPlan p = emb_plan(D, vocab);
-  if (seq + p.groups > 0x7fffffff) return nl_set_error(NL_EINVAL, "embedding_bwd: vocabulary too large");
+  const int64_t grid = seq + (int64_t)p.buckets * ((p.W + emb_rows(D) - 1) / emb_rows(D));
+  if (grid > 0x7fffffff) return nl_set_error(NL_EINVAL, "embedding_bwd: vocabulary too large");
   const int T = (int)T64;
   hipStream_t st = (hipStream_t)stream;
   int* counts = nullptr;
@@ -803,7 +949,14 @@ extern "C" int nl_embedding_bwd(void* stream, int batch, int seq, int D, int voc
                        offsets, lists);
   }
   // with no tokens every row of dtok is still written (zero): counts is not read then
-  hipLaunchKernelGGL(embed_bwd_kernel, dim3((unsigned)(seq + p.groups)), dim3(64), p.R * D * 4, st, batch, seq, D,
-                     ids, dx, dtok, vocab, p.R, p.W, counts, offsets, lists, dpos, accumulate_pos);
+  auto go = [&](auto f) {
+    f(st, grid, batch, seq, D, dx, dtok, vocab, p.W, counts, offsets, lists, dpos, accumulate_pos);
+  };
+  switch (emb_rows(D)) {
+    case 8: go(launch_embed_bwd<2, 8>); break;
+    case 4: go(launch_embed_bwd<4, 4>); break;
+    case 2: go(launch_embed_bwd<4, 2>); break;
+    default: go(launch_embed_bwd<4, 1>); break;
+  }
   return nl_check_launch("nl_embedding_bwd");
 }

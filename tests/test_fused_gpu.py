@@ -320,6 +320,38 @@ def test_embedding_bwd_sums_in_token_order(dev, pattern):
     assert np.array_equal(_np(dpos), ref_pos)
 
 
+@pytest.mark.parametrize("D", [4, 260, 512, 516, 1100, 2052, 4096])
+def test_embedding_bwd_text_frequencies_and_widths(dev, D):
+    """Ids with 1/rank frequencies (rows of hundreds of tokens beside empty
+    ones, buckets of more than one 512-entry chunk) at widths on both sides of
+    each column split: np.add.at's float32 sums, bit for bit, with dx on an
+    8-byte boundary only."""
+    import torch
+    from nlearn_amd import _lib
+
+    B, S, V = 5, 700, 411
+    rng = np.random.default_rng(D)
+    ids = np.minimum(np.exp(rng.random((B, S)) * np.log(V + 1.0)) - 1.0, V - 1).astype(np.int32)
+    dx = ops.bf16_round(rng.standard_normal((B, S, D)).astype(np.float32))
+    base = torch.empty(B * S * D + 4, dtype=torch.bfloat16, device=dev)
+    base[4:] = torch.from_numpy(dx.reshape(-1)).to(dev)
+    dtok = torch.full((V, D), float("nan"), device=dev)
+    dpos = torch.empty((S, D), device=dev)
+    wsb = int(_lib.load().nl_embedding_bwd_ws_bytes(B, S, D, V))
+    ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+    _lib.call("nl_embedding_bwd", torch.cuda.current_stream().cuda_stream, B, S, D, V,
+              torch.from_numpy(ids).to(dev).data_ptr(), base.data_ptr() + 8, dtok.data_ptr(), dpos.data_ptr(), 0,
+              ws.data_ptr(), wsb)
+    torch.cuda.synchronize()
+    ref = np.zeros((V, D), np.float32)
+    np.add.at(ref, ids.reshape(-1), dx.reshape(-1, D))
+    assert np.array_equal(_np(dtok), ref)
+    ref_pos = np.zeros((S, D), np.float32)
+    for b in range(B):
+        ref_pos += dx[b]
+    assert np.array_equal(_np(dpos), ref_pos)
+
+
 def test_embedding_invalid_ids_give_nan_rows(dev):
     import torch
     from nlearn_amd.kernels.fused import embedding
