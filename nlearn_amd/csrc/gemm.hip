@@ -23,6 +23,10 @@
 //     operand then arrives in 128-byte pieces of each row: when the previous
 //     kernel has just written it, it comes from DRAM, where 64-byte pieces
 //     (32-k stages) ran a third slower.
+//   * Products too small to fill the chip (a few thousand tokens) take 64 x 64
+//     tiles with 128-k stages, or 128 x 64 ones: they wait on the DMA round trip
+//     of each stage, so more, smaller workgroups and fewer stages are what
+//     helps. make_plan draws the lines, with the times on both sides.
 //   * 256 x 256 tiles (8 waves, the LM head) bound by the CU's global -> LDS
 //     path; in the weight-gradient (TN) form half of the waves issue each
 //     stage's DMA, so one wave per SIMD computes while the other queues loads.
@@ -36,6 +40,8 @@
 //   * Operands beyond the 2 GB reach of 32-bit buffer offsets are split on the
 //     host into sub-products that fit it (panels of M or N; chunks of K summed
 //     in the fp32 output).
+#include <type_traits>
+
 #include "common.h"
 
 namespace nl {
@@ -233,10 +239,11 @@ __device__ __forceinline__ void epilogue4_any(const GemmArgs& g, int64_t m, int 
 
 // K-major tiles keep CH = BKT/8 16-byte chunks per row; chunk kc of row r sits
 // at slot kc ^ kswz(r). Eight consecutive rows at one chunk (a fragment read)
-// land on distinct banks for CH = 8 and CH = 4.
+// land on distinct banks for CH = 16, CH = 8 and CH = 4.
 template <int CH>
 __device__ __forceinline__ int kswz(int r) {
-  if constexpr (CH == 8) return (r ^ (r >> 3)) & 7;
+  if constexpr (CH == 16) return r & 15;
+  else if constexpr (CH == 8) return (r ^ (r >> 3)) & 7;
   else return (r >> 1) & 3;
 }
 
@@ -245,7 +252,13 @@ __device__ __forceinline__ int kswz(int r) {
 // 4 (k & 3) maps those 16 (chunk, k) pairs to 16 distinct slots mod 16, i.e.
 // all 64 banks (rows are 256 or 512 bytes). The former 2k swizzle paired them
 // up: 2-way conflicts, measured as 28% of LDS cycles on the LM-head NN GEMM.
-__device__ __forceinline__ int mnswz(int k) { return (4 * k) & 15; }
+// A 64-wide tile's rows are 128 bytes, so even and odd k-rows already sit in
+// different halves of the banks and only k and k + 2 have to be told apart.
+template <int ROWS>
+__device__ __forceinline__ int mnswz(int k) {
+  if constexpr (ROWS == 64) return ((k >> 1) & 1) << 2;
+  else return (4 * k) & 15;
+}
 
 // Per-lane DMA offsets of one ROWS x BKT operand tile filled by NW waves.
 template <int ROWS, int BKT, bool KMAJ, int NW>
@@ -264,7 +277,7 @@ struct Dma {
       } else {
         constexpr int CPR = ROWS / 8, RPI = 64 / CPR;
         const int k = (i * NW + wave) * RPI + lane / CPR;
-        const int c = (lane % CPR) ^ mnswz(k);
+        const int c = (lane % CPR) ^ mnswz<ROWS>(k);
         voff[i] = (uint32_t)(((int64_t)k * ld + row0 + c * 8) * 2);
       }
     }
@@ -302,7 +315,7 @@ __device__ __forceinline__ void stage_masked(const uint16_t* __restrict__ P, int
       const int gk = k0 + k, gm = row0 + c * 8;
       u32x4 v = {0u, 0u, 0u, 0u};
       if (gk < k_lim) v = load8(P + (int64_t)gk * ld + gm, rows_lim - gm);
-      *reinterpret_cast<u32x4*>(lds + k * ROWS + ((c ^ mnswz(k)) << 3)) = v;
+      *reinterpret_cast<u32x4*>(lds + k * ROWS + ((c ^ mnswz<ROWS>(k)) << 3)) = v;
     }
   }
 }
@@ -325,7 +338,7 @@ struct Frag {
 #pragma unroll
       for (int rr = 0; rr < 2; ++rr) {
         const int k = 8 * g + 4 * rr + (j >> 2);  // + ks*16 (does not change the swizzle key)
-        off[rr] = k * ROWS + (((mn >> 3) ^ mnswz(k)) << 3) + (mn & 7);
+        off[rr] = k * ROWS + (((mn >> 3) ^ mnswz<ROWS>(k)) << 3) + (mn & 7);
       }
       sw = 0;
     }
@@ -376,28 +389,18 @@ __device__ __forceinline__ void ce_combine(float& m, float& s, float m2, float s
   m = mn;
 }
 
-// wait until at most `later` stages (IPS DMA ops each) of this wave are outstanding
-template <int IPS, int MAXL>
-__device__ __forceinline__ void wait_stage(int later) {
-  if constexpr (MAXL <= 0) {
-    wait_vm<0>();
-  } else {
-    if (later >= MAXL) wait_vm<MAXL * IPS>();
-    else wait_stage<IPS, MAXL - 1>(later);
-  }
-}
-
-template <int BM, int BN, int BKT, int S, bool A_KMAJ, bool B_KMAJ, typename OutT, int EPI>
+template <int BM, int BN, int BKT, bool A_KMAJ, bool B_KMAJ, typename OutT, int EPI>
 __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
                              (BM * BN >= 65536) ? 1 : 2) void gemm2_kernel(GemmArgs g) {
   // 256 x 256 tiles run 8 waves (2 x 4), the others 4 (2 x 2); every wave
-  // owns a WTM x 64 block of the tile.
+  // owns a WTM x WTN block of the tile.
   constexpr bool kHuge = BM * BN >= 65536;
   constexpr int NWV = kHuge ? 8 : 4;
   constexpr int NT = 64 * NWV;
-  constexpr int WNW = BN / 64, WMW = NWV / WNW;
+  constexpr int WTN = BN == 64 ? 32 : 64;
+  constexpr int WNW = BN / WTN, WMW = NWV / WNW;
   static_assert(WNW * WMW == NWV, "wave layout");
-  constexpr int WTM = BM / WMW, WTN = 64;
+  constexpr int WTM = BM / WMW;
   constexpr int FM = WTM / 32, FN = WTN / 32;
   constexpr int STAGE = (BM + BN) * BKT;  // elements per stage
   // After the K loop the same LDS holds the epilogue: four 8 KB store slabs at
@@ -405,13 +408,11 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
   // pre-activation tile (32 KB).
   constexpr bool kBias = EPI == NL_EPI_BIAS || EPI == NL_EPI_BIAS_GELU;
   constexpr bool kAux = EPI == NL_EPI_DGELU;
-  static_assert(S == 2 || S == 3, "two or three pipeline stages");
   // Each pipeline stage is its own LDS object: the compiler can then prove that
   // the DMA filling one stage does not alias the reads of another and does not
   // make those reads wait for it.
   __shared__ __attribute__((aligned(16))) uint16_t st0[STAGE];
   __shared__ __attribute__((aligned(16))) uint16_t st1[STAGE];
-  __shared__ __attribute__((aligned(16))) uint16_t st2[S > 2 ? STAGE : 8];
   // Epilogue LDS: four 8 KB store slabs (in the stage buffers), the bias
   // columns (1 KB) and, for the GELU backward, the saved pre-activation tile
   // (32 KB: the second stage buffer when stages are that large).
@@ -465,12 +466,11 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
   // bandwidth); this way one of the two computes meanwhile. Measured at
   // 512 x 50257 x 16384: 771-777 -> 737-744 us.
   // (Slower for the NT form, 672-695 -> 694-708 us, and for 128 x 128 tiles.)
-  constexpr int DNW = (!A_KMAJ && !B_KMAJ && kHuge && S == 2) ? NWV / 2 : NWV;
+  constexpr int DNW = (!A_KMAJ && !B_KMAJ && kHuge) ? NWV / 2 : NWV;
   Dma<BM, BKT, A_KMAJ, DNW> da;
   Dma<BN, BKT, B_KMAJ, DNW> db;
   da.init(m0, g.lda, wave % DNW, lane);
   db.init(n0, g.ldb, wave % DNW, lane);
-  constexpr int IPS = Dma<BM, BKT, A_KMAJ, DNW>::INSTR + Dma<BN, BKT, B_KMAJ, DNW>::INSTR;  // DMA ops per stage per issuing wave
 
   Frag<BM, BKT, A_KMAJ> fa[FM];
   Frag<BN, BKT, B_KMAJ> fb[FN];
@@ -487,10 +487,35 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
+  constexpr bool kFewMfma = FM * FN <= 2;
   bf16x8 af[2][FM], bfr[2][FN];
   auto compute = [&](const uint16_t* sb) __attribute__((always_inline)) {
     const uint16_t* As = sb;
     const uint16_t* Bs = sb + BM * BKT;
+    if constexpr (kFewMfma) {
+      // one or two MFMAs per k16 step cannot cover a fragment read: every read of
+      // the stage is queued before its first MFMA, so one LDS latency is exposed
+      // per stage and not one per step
+      constexpr int KS = BKT / 16;
+      bf16x8 sa[KS][FM], sbf[KS][FN];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i) sa[ks][i] = fa[i].read(As, ks, lane);
+#pragma unroll
+        for (int j = 0; j < FN; ++j) sbf[ks][j] = fb[j].read(Bs, ks, lane);
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) acc[i][j] = mfma32(sbf[ks][j], sa[ks][i], acc[i][j]);
+      constexpr int R = FM * (A_KMAJ ? 1 : 2) + FN * (B_KMAJ ? 1 : 2);
+      __builtin_amdgcn_sched_group_barrier(0x100, R * KS, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, FM * FN * KS, 0);
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < FM; ++i) af[0][i] = fa[i].read(As, 0, lane);
 #pragma unroll
@@ -523,40 +548,25 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
     }
   };
 
-  // S-stage pipeline, unrolled by S so that every buffer is a fixed LDS object.
-  // Step kt: wait until this wave's DMA of stage kt has landed (later stages
-  // may stay in flight), barrier (stage kt complete for all waves, all waves
-  // done with stage kt-1), start the DMA of stage kt+S-1 into the buffer of
-  // stage kt-1, compute stage kt. With three stages the barrier is a bare
-  // s_barrier (a memory clobber for the compiler): __syncthreads would also
-  // wait for the DMA still in flight.
+  // Two-stage pipeline, unrolled so that both buffers are fixed LDS objects.
+  // Step kt: wait until this wave's DMA of stage kt has landed, barrier (stage
+  // kt complete for all waves, all waves done with stage kt-1), start the DMA
+  // of stage kt+1 into the buffer of stage kt-1, compute stage kt.
   auto step = [&](uint16_t* cur, uint16_t* nxt, int kt) __attribute__((always_inline)) {
-    wait_stage<IPS, S - 2>(min(S - 2, nfull - 1 - kt));
-    if constexpr (S == 2) __syncthreads();
-    else asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // this wave's LDS reads done
-    if (kt + S - 1 < nfull) issue(nxt, kt + S - 1);
+    wait_vm<0>();
+    __syncthreads();
+    if (kt + 1 < nfull) issue(nxt, kt + 1);
     compute(cur);
   };
   if (nfull > 0) issue(st0, 0);
-  if (S > 2 && nfull > 1) issue(st1, 1);
-  if constexpr (S == 2) {
-    for (int kt = 0; kt < nfull; kt += 2) {
-      step(st0, st1, kt);
-      if (kt + 1 >= nfull) break;
-      step(st1, st0, kt + 1);
-    }
-  } else {
-    for (int kt = 0; kt < nfull; kt += 3) {
-      step(st0, st2, kt);
-      if (kt + 1 >= nfull) break;
-      step(st1, st0, kt + 1);
-      if (kt + 2 >= nfull) break;
-      step(st2, st1, kt + 2);
-    }
+  for (int kt = 0; kt < nfull; kt += 2) {
+    step(st0, st1, kt);
+    if (kt + 1 >= nfull) break;
+    step(st1, st0, kt + 1);
   }
   if (tail) {
     __syncthreads();
-    uint16_t* sb = (nfull % S) == 0 ? st0 : (nfull % S) == 1 ? st1 : st2;
+    uint16_t* sb = nfull % 2 == 0 ? st0 : st1;
     const int kt0 = kbeg + nfull * BKT;
     stage_masked<BM, BKT, A_KMAJ, NT>(g.A, g.lda, m0, g.M, kt0, kend, sb, tid);
     stage_masked<BN, BKT, B_KMAJ, NT>(g.B, g.ldb, n0, g.N, kt0, kend, sb + BM * BKT, tid);
@@ -674,7 +684,9 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
   // into LDS by DMA before the first store: a wait on a vector load also waits
   // for every earlier store, so loads mixed into the store stream would
   // serialise it. The operand tiles' LDS is free once all waves pass the barrier.
-  static_assert((!kBias && !kAux) || (BM == 128 && BN == 128), "the staged epilogue assumes 128 x 128 tiles");
+  static_assert(!kBias || BN <= 256, "the bias of a tile's columns is one DMA instruction");
+  constexpr int ACPR = BN / 8;  // 16-byte chunks per row of the aux tile
+  static_assert(!kAux || ACPR <= 64, "whole rows per DMA instruction");
   uint16_t* const xlds = kAuxInSt1 ? st1 : aux_lds;
   const float* sbias = sbias_lds;
   __syncthreads();
@@ -687,14 +699,14 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
                                                  0);
       }
     } else {
-      // aux tile [128][128] bf16: row r at r*256 bytes, 16-byte chunk c at slot c ^ (r & 15)
+      // aux tile [BM][BN] bf16: row r at r*2*BN bytes, 16-byte chunk c at slot c ^ (r & (ACPR - 1))
       const uint32_t aux_bytes = (uint32_t)(((int64_t)g.M * g.ldaux) * 2);
       const __amdgpu_buffer_rsrc_t raux = make_rsrc(g.aux, aux_bytes);
 #pragma unroll
       for (int i = 0; i < BM * BN * 2 / 1024 / NWV; ++i) {
-        const int blk = i * NWV + wave;            // 1 KB block = 4 rows
-        const int r = blk * 4 + (lane >> 4);
-        const int c = (lane & 15) ^ (r & 15);
+        const int blk = i * NWV + wave;            // 1 KB block = 64 / ACPR rows
+        const int r = blk * (64 / ACPR) + lane / ACPR;
+        const int c = (lane % ACPR) ^ (r & (ACPR - 1));
         const uint32_t off = (uint32_t)(((int64_t)(m0 + r) * g.ldaux + n0 + c * 8) * 2);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(raux, (lds_void*)(xlds + blk * 512), 16, off, 0, 0, 0);
       }
@@ -764,7 +776,7 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
     u32x2 a = {0u, 0u};
     if constexpr (kAux) {
       const int ml = wm * WTM + i * 32 + frow;
-      a = *reinterpret_cast<const u32x2*>(xlds + ml * 128 + (((nl >> 3) ^ (ml & 15)) << 3) + (nl & 7));
+      a = *reinterpret_cast<const u32x2*>(xlds + ml * BN + (((nl >> 3) ^ (ml & (ACPR - 1))) << 3) + (nl & 7));
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -1131,17 +1143,24 @@ __global__ __launch_bounds__(NWV * 64, NWV == 8 ? 1 : 2) void gemm_persist_kerne
 
 // Explicit instantiations: every (layout, output, epilogue) combination the
 // dispatcher can launch gets its host stub emitted.
-#define NL_I(AK, BKM, T, E) template __global__ void gemm2_kernel<128, 128, 64, 2, AK, BKM, T, E>(GemmArgs);
+#define NL_I(AK, BKM, T, E) template __global__ void gemm2_kernel<128, 128, 64, AK, BKM, T, E>(GemmArgs);
 #define NL_I4(T, E) NL_I(true, false, T, E) NL_I(true, true, T, E) NL_I(false, false, T, E) NL_I(false, true, T, E)
 #define NL_I8(E) NL_I4(float, E) NL_I4(uint16_t, E)
+#define NL_S(BM, BN, BKT, AK, BKM, E)                                           \
+  template __global__ void gemm2_kernel<BM, BN, BKT, AK, BKM, float, E>(GemmArgs); \
+  template __global__ void gemm2_kernel<BM, BN, BKT, AK, BKM, uint16_t, E>(GemmArgs);
+#define NL_S3(BM, BN, BKT, E) NL_S(BM, BN, BKT, true, false, E) NL_S(BM, BN, BKT, true, true, E) NL_S(BM, BN, BKT, false, false, E)
+#define NL_SALL(BM, BN, BKT) NL_S3(BM, BN, BKT, NL_EPI_NONE) NL_S3(BM, BN, BKT, NL_EPI_BIAS) NL_S3(BM, BN, BKT, NL_EPI_BIAS_GELU) NL_S3(BM, BN, BKT, NL_EPI_DGELU)
+NL_SALL(64, 64, 128)
+NL_SALL(128, 64, 64)
 NL_I8(NL_EPI_NONE)
 NL_I8(NL_EPI_BIAS)
 NL_I8(NL_EPI_BIAS_GELU)
 NL_I8(NL_EPI_DGELU)
-template __global__ void gemm2_kernel<256, 128, 32, 2, true, false, float, NL_EPI_NONE>(GemmArgs);
-template __global__ void gemm2_kernel<256, 256, 64, 2, true, false, uint16_t, kEpiCeStats>(GemmArgs);
-template __global__ void gemm2_kernel<256, 256, 64, 2, true, false, uint16_t, kEpiCeGrad>(GemmArgs);
-template __global__ void gemm2_kernel<256, 256, 64, 2, true, true, float, NL_EPI_NONE>(GemmArgs);
+template __global__ void gemm2_kernel<256, 128, 32, true, false, float, NL_EPI_NONE>(GemmArgs);
+template __global__ void gemm2_kernel<256, 256, 64, true, false, uint16_t, kEpiCeStats>(GemmArgs);
+template __global__ void gemm2_kernel<256, 256, 64, true, false, uint16_t, kEpiCeGrad>(GemmArgs);
+template __global__ void gemm2_kernel<256, 256, 64, true, true, float, NL_EPI_NONE>(GemmArgs);
 template __global__ void gemm_persist_kernel<true, true, float>(GemmArgs);
 template __global__ void gemm_persist_kernel<true, true, uint16_t>(GemmArgs);
 template __global__ void gemm_persist_kernel<true, false, float>(GemmArgs);
@@ -1158,14 +1177,17 @@ template __global__ void gemm_persist_kernel<true, true, float, 128, 128, 4, NL_
 template __global__ void gemm_persist_kernel<true, true, uint16_t, 128, 128, 4, NL_EPI_BIAS>(GemmArgs);
 template __global__ void gemm_persist_kernel<true, false, uint16_t, 128, 128, 4, NL_EPI_BIAS_GELU>(GemmArgs);
 template __global__ void gemm_persist_kernel<true, true, uint16_t, 128, 128, 4, NL_EPI_BIAS_GELU>(GemmArgs);
-template __global__ void gemm2_kernel<256, 256, 64, 2, true, true, uint16_t, NL_EPI_NONE>(GemmArgs);
-template __global__ void gemm2_kernel<256, 256, 64, 2, true, false, float, NL_EPI_NONE>(GemmArgs);
-template __global__ void gemm2_kernel<256, 256, 64, 2, true, false, uint16_t, NL_EPI_NONE>(GemmArgs);
-template __global__ void gemm2_kernel<256, 256, 64, 2, false, false, float, NL_EPI_NONE>(GemmArgs);
-template __global__ void gemm2_kernel<256, 256, 64, 2, false, false, uint16_t, NL_EPI_NONE>(GemmArgs);
-template __global__ void gemm2_kernel<256, 128, 32, 2, true, false, uint16_t, NL_EPI_NONE>(GemmArgs);
-template __global__ void gemm2_kernel<256, 128, 32, 2, false, false, float, NL_EPI_NONE>(GemmArgs);
-template __global__ void gemm2_kernel<256, 128, 32, 2, false, false, uint16_t, NL_EPI_NONE>(GemmArgs);
+template __global__ void gemm2_kernel<256, 256, 64, true, true, uint16_t, NL_EPI_NONE>(GemmArgs);
+template __global__ void gemm2_kernel<256, 256, 64, true, false, float, NL_EPI_NONE>(GemmArgs);
+template __global__ void gemm2_kernel<256, 256, 64, true, false, uint16_t, NL_EPI_NONE>(GemmArgs);
+template __global__ void gemm2_kernel<256, 256, 64, false, false, float, NL_EPI_NONE>(GemmArgs);
+template __global__ void gemm2_kernel<256, 256, 64, false, false, uint16_t, NL_EPI_NONE>(GemmArgs);
+template __global__ void gemm2_kernel<256, 128, 32, true, false, uint16_t, NL_EPI_NONE>(GemmArgs);
+template __global__ void gemm2_kernel<256, 128, 32, false, false, float, NL_EPI_NONE>(GemmArgs);
+template __global__ void gemm2_kernel<256, 128, 32, false, false, uint16_t, NL_EPI_NONE>(GemmArgs);
+#undef NL_SALL
+#undef NL_S3
+#undef NL_S
 #undef NL_I8
 #undef NL_I4
 #undef NL_I
@@ -1212,7 +1234,6 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmArgs g, int spli
   }
 }
 
-// Tile configuration and K split of one product (shared by the workspace query).
 // Compute units of the current device (cached per device).
 int cu_count() {
   static int cached[64] = {0};
@@ -1226,8 +1247,11 @@ int cu_count() {
   return cached[dev];
 }
 
+enum Tile { kTile64, kTile128x64, kTile128, kTile256x128, kTile256 };
+
+// Tile configuration and K split of one product (shared by the workspace query).
 struct Plan {
-  int big;     // 1: 256 x 128 tiles (the very large products), 0: 128 x 128
+  Tile tile;
   int tiles;
   int splits;
   int k_chunk;
@@ -1237,7 +1261,7 @@ struct Plan {
 
 Plan make_plan(int opA, int opB, int M, int N, int K, int epi) {
   Plan p;
-  p.big = 0;
+  p.tile = kTile128;
   p.tiles = (int)((int64_t)((M + 127) / 128) * ((N + 127) / 128));
   p.splits = 1;
   p.k_chunk = K > 0 ? K : 1;
@@ -1271,7 +1295,7 @@ Plan make_plan(int opA, int opB, int M, int N, int K, int epi) {
   // beat 128 x 128 on the LM head (TN 16384-deep: ~15%), lose on the FFN sizes.
   if (p.splits == 1 && opB == NL_OP_N && epi == NL_EPI_NONE &&
       ((opA == NL_OP_T && p.tiles >= 1024) || (opA == NL_OP_N && p.tiles >= 8192))) {
-    p.big = 1;
+    p.tile = kTile256x128;
     p.tiles = (int)((int64_t)((M + 255) / 256) * ((N + 127) / 128));
   }
   // 256 x 256 tiles (8 waves of 128 x 64, 64-k stages) for products of
@@ -1281,7 +1305,7 @@ Plan make_plan(int opA, int opB, int M, int N, int K, int epi) {
   // 896 us, NT 1186 -> 897 us, TN 931 -> 811 us.
   // One workgroup per CU, so a short grid splits K up to 256 workgroups.
   if (epi == NL_EPI_NONE && !(opA == NL_OP_T && opB == NL_OP_T) && 2.0 * M * N * K >= 1e11) {
-    p.big = 2;
+    p.tile = kTile256;
     p.tiles = (int)((int64_t)((M + 255) / 256) * ((N + 255) / 256));
     p.splits = 1;
     p.k_chunk = K;
@@ -1291,6 +1315,45 @@ Plan make_plan(int opA, int opB, int M, int N, int K, int epi) {
       chunk = (chunk + BK - 1) / BK * BK;
       p.k_chunk = chunk;
       p.splits = (K + chunk - 1) / chunk;
+    }
+  }
+  // Products too small to give every CU two 128 x 128 tiles (a few hundred to a
+  // few thousand tokens): they wait on their k stages, one DMA round trip after
+  // the other, and on the split's second launch, not on MFMAs. 64 x 64 tiles
+  // with 128-k stages (half the barriers and round trips, 64 KB of LDS) put four
+  // times the workgroups on the chip and need no split up to K = 2048. Measured
+  // (us, operands in the caches; 128 x 128 -> these):
+  //   NN 200 x 512 x 512     6.8 -> 3.9    NN 4096 x 512 x 512   7.3 -> 5.6
+  //   NN 2048 x 512 x 2048  20.3 -> 9.1    NN 4096 x 512 x 2048 24.3 -> 12.4
+  //   TN 512 x 2048 x 2048  19.5 -> 9.7    TN 512 x 512 x 4096  15.3 -> 10.2
+  // The bound on their number is where two rounds of them lose: NN 2048 x 1536
+  // x 512 (768 tiles) 7.5 -> 8.1, 6000 x 512 x 2048 (752) 24.1 against 20.8 with
+  // 128 x 64 tiles. Those take over up to 256 tiles of 128 x 128 (2048 x 2048 x
+  // 512 10.3 -> 9.1, 8192 x 512 x 2048 23.4 -> 20.9, 1000 x 4096 x 1024 15.4 ->
+  // 13.1; beyond, 12000 x 512 x 2048 28.0 -> 31.8). Long reductions run on
+  // 64 x 64 tiles, split, only over the smallest outputs (TN 512 x 512 x 16384
+  // 22.1 -> 19.9, NT 256 x 512 x 50256 38.7 -> 31.5; but 1024 x 512 x 50256
+  // 89.6 -> 91.3).
+  const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+  const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+  if (!(opA == NL_OP_T && opB == NL_OP_T) && K > 0) {
+    if (t64 <= (K <= 4096 ? 512 : 64)) {
+      p.tile = kTile64;
+      p.tiles = (int)t64;
+      p.splits = 1;
+      p.k_chunk = K;
+      const int per = K <= 4096 ? 1024 : 2048;
+      const int sp = std::min(512 / p.tiles, (K + per - 1) / per);
+      if (K > 2048 && sp > 1) {
+        const int chunk = ((K + sp - 1) / sp + 127) / 128 * 128;
+        p.k_chunk = chunk;
+        p.splits = (K + chunk - 1) / chunk;
+      }
+    } else if (t128 <= 256 && K <= 4096) {
+      p.tile = kTile128x64;
+      p.tiles = (int)((int64_t)((M + 127) / 128) * ((N + 63) / 64));
+      p.splits = 1;
+      p.k_chunk = K;
     }
   }
   p.ldw = ((int64_t)N + 7) / 8 * 8;
@@ -1312,7 +1375,7 @@ void launch_cfg(GemmArgs g, const Plan& p, hipStream_t st) {
   // 66 -> 58 us; in the training step 52-59 -> 42-47 us).
   auto launch2 = [&](int grid) {
     if constexpr (AK || !BK_) {
-      if (p.big == 2) {
+      if (p.tile == kTile256) {
         // short-K products without a split: one persistent workgroup per CU
         if (!g.ws && g.beta == 0.f && g.K % 128 == 0 && g.K <= 4096) {
           const int cus = cu_count();
@@ -1321,17 +1384,35 @@ void launch_cfg(GemmArgs g, const Plan& p, hipStream_t st) {
           hipLaunchKernelGGL((gemm_persist_kernel<AK, BK_, OutT>), dim3(G), dim3(512), 0, st, g);
           return;
         }
-        hipLaunchKernelGGL((gemm2_kernel<256, 256, 64, 2, AK, BK_, OutT, NL_EPI_NONE>), dim3(grid), dim3(512), 0, st, g);
+        hipLaunchKernelGGL((gemm2_kernel<256, 256, 64, AK, BK_, OutT, NL_EPI_NONE>), dim3(grid), dim3(512), 0, st, g);
         return;
       }
     }
     if constexpr (!BK_) {
-      if (p.big == 1) {
-        hipLaunchKernelGGL((gemm2_kernel<256, 128, 32, 2, AK, BK_, OutT, NL_EPI_NONE>), dim3(grid), dim3(256), 0, st, g);
+      if (p.tile == kTile256x128) {
+        hipLaunchKernelGGL((gemm2_kernel<256, 128, 32, AK, BK_, OutT, NL_EPI_NONE>), dim3(grid), dim3(256), 0, st, g);
         return;
       }
     }
-    constexpr int BKT = 64, NS = 2;
+    if constexpr (AK || !BK_) {
+      if (p.tile == kTile64 || p.tile == kTile128x64) {
+        auto go = [&](auto e) {
+          constexpr int E = decltype(e)::value;
+          if (p.tile == kTile64)
+            hipLaunchKernelGGL((gemm2_kernel<64, 64, 128, AK, BK_, OutT, E>), dim3(grid), dim3(256), 0, st, g);
+          else
+            hipLaunchKernelGGL((gemm2_kernel<128, 64, 64, AK, BK_, OutT, E>), dim3(grid), dim3(256), 0, st, g);
+        };
+        switch (g.ws ? NL_EPI_NONE : g.epi) {
+          case NL_EPI_BIAS: go(std::integral_constant<int, NL_EPI_BIAS>{}); break;
+          case NL_EPI_BIAS_GELU: go(std::integral_constant<int, NL_EPI_BIAS_GELU>{}); break;
+          case NL_EPI_DGELU: go(std::integral_constant<int, NL_EPI_DGELU>{}); break;
+          default: go(std::integral_constant<int, NL_EPI_NONE>{});
+        }
+        return;
+      }
+    }
+    constexpr int BKT = 64;
     // Short-K products with at least 4 tiles per workgroup and no epilogue or a
     // bias / bias + GELU one (QKV and FFN-up): the persistent kernel, two
     // 128 x 128 workgroups per CU, each loading its next tile's first stage
@@ -1364,18 +1445,18 @@ void launch_cfg(GemmArgs g, const Plan& p, hipStream_t st) {
     const int epi = g.ws ? NL_EPI_NONE : g.epi;
     switch (epi) {
       case NL_EPI_BIAS:
-        hipLaunchKernelGGL((gemm2_kernel<128, 128, BKT, NS, AK, BK_, OutT, NL_EPI_BIAS>), dim3(grid), dim3(256), 0, st, g);
+        hipLaunchKernelGGL((gemm2_kernel<128, 128, BKT, AK, BK_, OutT, NL_EPI_BIAS>), dim3(grid), dim3(256), 0, st, g);
         break;
       case NL_EPI_BIAS_GELU:
-        hipLaunchKernelGGL((gemm2_kernel<128, 128, BKT, NS, AK, BK_, OutT, NL_EPI_BIAS_GELU>), dim3(grid), dim3(256), 0,
+        hipLaunchKernelGGL((gemm2_kernel<128, 128, BKT, AK, BK_, OutT, NL_EPI_BIAS_GELU>), dim3(grid), dim3(256), 0,
                            st, g);
         break;
       case NL_EPI_DGELU:
-        hipLaunchKernelGGL((gemm2_kernel<128, 128, BKT, NS, AK, BK_, OutT, NL_EPI_DGELU>), dim3(grid), dim3(256), 0, st,
+        hipLaunchKernelGGL((gemm2_kernel<128, 128, BKT, AK, BK_, OutT, NL_EPI_DGELU>), dim3(grid), dim3(256), 0, st,
                            g);
         break;
       default:
-        hipLaunchKernelGGL((gemm2_kernel<128, 128, BKT, NS, AK, BK_, OutT, NL_EPI_NONE>), dim3(grid), dim3(256), 0, st, g);
+        hipLaunchKernelGGL((gemm2_kernel<128, 128, BKT, AK, BK_, OutT, NL_EPI_NONE>), dim3(grid), dim3(256), 0, st, g);
     }
   };
   if (p.splits > 1) {
@@ -1532,7 +1613,7 @@ void launch_lce(GemmArgs g, hipStream_t st) {
   g.tiles = (int)((int64_t)((g.M + kLceTile - 1) / kLceTile) * lce_tiles_n(g.N));
   g.k_chunk = g.K;
   g.ws = nullptr;
-  hipLaunchKernelGGL((gemm2_kernel<kLceTile, kLceTile, 64, 2, true, false, uint16_t, EPI>), dim3(g.tiles), dim3(512),
+  hipLaunchKernelGGL((gemm2_kernel<kLceTile, kLceTile, 64, true, false, uint16_t, EPI>), dim3(g.tiles), dim3(512),
                      0, st, g);
 }
 

@@ -247,6 +247,46 @@ def test_gemm_tall_tile_path_exact_small_integers(dev, opA, M, N, K):
     assert np.array_equal(got, A[rows] @ B)
 
 
+@pytest.mark.parametrize("opA,opB", [("N", "N"), ("N", "T"), ("T", "N")])
+@pytest.mark.parametrize("M,N,K", [
+    (63, 65, 128), (64, 64, 127), (129, 190, 257), (4096, 512, 130),   # 64 x 64 tiles (the last: as many as they take)
+    (70, 66, 2049), (130, 200, 5000),                                  # ... split over K
+    (2000, 1100, 192), (8130, 500, 65), (2048, 2047, 64),              # 128 x 64 tiles
+    (2100, 2100, 200)])                                                # 128 x 128 tiles, one pass
+def test_gemm_small_product_tiles(dev, opA, opB, M, N, K):
+    """Tile edges and K remainders of the tiles for products that do not fill
+    the chip, and of the next larger ones: fp32 and bf16 outputs, beta, and the
+    bias / GELU' epilogues (after the reduction where K is split). Small
+    integers: products and sums are exact in fp32."""
+    import torch
+    from nlearn_amd.kernels.gemm import EPI_BIAS, EPI_DGELU, gemm_raw, padded_empty
+    from oracle import model_np as om
+
+    rng = np.random.default_rng(M + 7 * N + 13 * K)
+    A = rng.integers(-2, 3, (K, M) if opA == "T" else (M, K)).astype(np.float32)
+    B = rng.integers(-2, 3, (N, K) if opB == "T" else (K, N)).astype(np.float32)
+    ref = ops.gemm(A, B, opA, opB).astype(np.float32)
+    Ad, Bd = _dev_bf16(A, dev), _dev_bf16(B, dev)
+    bias = (rng.integers(-20, 21, N) / 4).astype(np.float32)
+    u = ops.bf16_round(rng.standard_normal((M, N)).astype(np.float32))
+    ud = padded_empty(M, N, torch.bfloat16, dev)
+    ud.copy_(_dev_bf16(u, dev))
+    c0 = padded_empty(M, N, torch.float32, dev)
+    c0.fill_(3.0)
+    f = gemm_raw(Ad, Bd, opA, opB)
+    b = gemm_raw(Ad, Bd, opA, opB, out_dtype=torch.bfloat16)
+    gemm_raw(Ad, Bd, opA, opB, out=c0, beta=2.0)
+    eb = gemm_raw(Ad, Bd, opA, opB, out_dtype=torch.bfloat16, epi=EPI_BIAS, bias=torch.from_numpy(bias).to(dev))
+    ed = gemm_raw(Ad, Bd, opA, opB, alpha=0.25, epi=EPI_DGELU, aux=ud)
+    torch.cuda.synchronize()
+    assert np.array_equal(_np(f), ref)
+    assert np.array_equal(_np(b), ops.bf16_round(ref))
+    assert np.array_equal(_np(c0), ref + 6.0)
+    assert np.array_equal(_np(eb), ops.bf16_round(ref + bias))
+    _, t = om._gelu(u.astype(np.float64))
+    assert rel_l2(_np(ed), om._gelu_bwd(0.25 * ref, u.astype(np.float64), t)) <= 1e-5   # as the epilogue test's bound
+
+
 @pytest.mark.parametrize("opB,M,N,K,out", [("N", 4100, 4000, 128, "f32"), ("N", 4100, 4000, 256, "bf16"),
                                            ("T", 4097, 4033, 384, "f32"), ("T", 16384, 2048, 512, "bf16"),
                                            ("N", 16384, 1536, 512, "bf16")])
