@@ -106,9 +106,9 @@ class KernelProbe:
             B, H, S, D = args[1:5]
             f = 2.0 * B * H * S * S * D if args[6] else 4.0 * B * H * S * S * D
             return f"flash_bwd_{B * H}x{S}x{D}", 2.5 * f, "flops"
-        # the training step launches the backward's kernels one by one (dQ on a
-        # second stream): executed products per kernel, S = QK^T and dP = dO V^T
-        # counted in both (dK/dV: S, dP, dV, dK; dQ: S, dP, dQ)
+        # the backward's kernels launched one by one: executed products per
+        # kernel, S = QK^T and dP = dO V^T counted in both (dK/dV: S, dP, dV, dK;
+        # dQ: S, dP, dQ)
         if name in ("nl_flash_attention_bwd_dkdv", "nl_flash_attention_bwd_dq"):
             B, H, S, D = args[1:5]
             f = 2.0 * B * H * S * S * D if args[6] else 4.0 * B * H * S * S * D

@@ -187,7 +187,7 @@ int nl_flash_attention_bwd_dkdv(void* stream, int batch, int heads, int seq, int
                                 nl_bf16* dK, nl_attn_stride sdk,
                                 nl_bf16* dV, nl_attn_stride sdv);
 
-/* Whole backward (preprocess + dK/dV + dQ) in one call. `ws` is a caller-owned
+/* Whole backward (D, dK/dV and dQ) in one call. `ws` is a caller-owned
  * device workspace of nl_flash_attention_bwd_ws_bytes() bytes (holds D).
  * Replaces _flash_bwd_rule (attention.py:111-128). */
 size_t nl_flash_attention_bwd_ws_bytes(int batch, int heads, int seq);

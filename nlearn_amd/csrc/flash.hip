@@ -28,6 +28,10 @@
 //     loads are in flight while the current one is consumed.
 //   * Causal work skipping per wave; fully masked waves only join the barriers.
 //     The heaviest tiles are launched first.
+//   * Few tiles (tile_grid): two wave groups per workgroup, 64 rows, each group
+//     every other block of the streamed side with buffers of its own; their
+//     partial results are combined in LDS. What bounds such a call is the chain
+//     of blocks of its longest tile on a chip that is not full.
 #include <type_traits>
 #include <atomic>
 #include <mutex>
@@ -142,14 +146,14 @@ __device__ __forceinline__ int swz_of(int k) {
 }
 
 // DMA rows row0 .. row0+63 (row stride ld elements) of the buffer into a tile:
-// 4 waves x 2 instructions x 64 lanes x 16 bytes. Rows past the buffer's end
-// read as zero.
-template <int W = kBoth>
+// NW waves x 8 / NW instructions x 64 lanes x 16 bytes. Rows past the buffer's
+// end read as zero.
+template <int W, int NW>
 __device__ __forceinline__ void dma_tile(__amdgpu_buffer_rsrc_t rs, uint16_t* lds, int row0, int64_t ld, int wave,
                                          int lane) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int blk = i * 4 + wave;           // 1 KB of the tile = 8 rows
+  for (int i = 0; i < 8 / NW; ++i) {
+    const int blk = i * NW + wave;          // 1 KB of the tile = 8 rows
     const int u = blk * 64 + lane;          // destination chunk
     const int r = u >> 3, slot = u & 7;
     const int c = slot ^ swz_of<W>(r);
@@ -249,21 +253,24 @@ __device__ __forceinline__ void store_rows_staged(uint16_t* slab, const f32x16 a
 // ---------------------------------------------------------------------------
 // forward
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads, 4) void flash_fwd_kernel(FwdArgs a) {
-  // double-buffered K and V blocks; every buffer its own
+template <int KS>
+__global__ __launch_bounds__(kThreads, KS == 1 ? 4 : 2) void flash_fwd_kernel(FwdArgs a) {
+  constexpr int ROWS = kRows / KS, NW = 4 / KS, TILE = kBlk * kD;
+  // double-buffered K and V blocks of each wave group; every buffer its own
   // LDS object so the DMA of block kb+1 never makes the reads of block kb wait
-  __shared__ __attribute__((aligned(16))) uint16_t sK0[kBlk * kD];
-  __shared__ __attribute__((aligned(16))) uint16_t sK1[kBlk * kD];
-  __shared__ __attribute__((aligned(16))) uint16_t sV0[kBlk * kD];
-  __shared__ __attribute__((aligned(16))) uint16_t sV1[kBlk * kD];
+  __shared__ __attribute__((aligned(16))) uint16_t sK0[KS * TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t sK1[KS * TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t sV0[KS * TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t sV1[KS * TILE];
   const int S = a.S;
-  const int nqt = (S + kRows - 1) / kRows;
+  const int nqt = (S + ROWS - 1) / ROWS;
   const TileCoord tc = tile_coord(a.H, a.B);
   const int qt = nqt - 1 - tc.rank;  // heaviest (latest) query tiles first
   const int h = tc.h, b = tc.b;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = KS == 1 ? 0 : wave / NW, wq = KS == 1 ? wave : wave % NW;  // key group, wave within it
   const int g = lane >> 5, l32 = lane & 31;
-  const int qw0 = qt * kRows + wave * 32;  // first query of this wave
+  const int qw0 = qt * ROWS + wq * 32;     // first query of this wave
   const int q = qw0 + l32;                 // this lane's query
   const bool qvalid = q < S;
 
@@ -274,14 +281,17 @@ __global__ __launch_bounds__(kThreads, 4) void flash_fwd_kernel(FwdArgs a) {
     for (int ks = 0; ks < 4; ++ks) qf[ks] = global_frag(qp + ks * 16 + g * 8, qvalid);
   }
 
-  const int kend_wg = a.causal ? min(S, qt * kRows + kRows) : S;
+  const int kend_wg = a.causal ? min(S, qt * ROWS + ROWS) : S;
   const int kend_w = a.causal ? min(S, qw0 + 32) : S;
   const int nkb = (kend_wg + kBlk - 1) / kBlk;
+  const int nit = (nkb + KS - 1) / KS;  // group grp takes blocks it * KS + grp
   const __amdgpu_buffer_rsrc_t rk = head_rsrc(a.k.at(b, h, 0), S, a.k.s.row);
   const __amdgpu_buffer_rsrc_t rv = head_rsrc(a.v.at(b, h, 0), S, a.v.s.row);
-  auto issue = [&](uint16_t* sk, uint16_t* sv, int kb) {
-    dma_tile<kAlongRows>(rk, sk, kb * kBlk, a.k.s.row, wave, lane);
-    dma_tile<kDownCols>(rv, sv, kb * kBlk, a.v.s.row, wave, lane);
+  auto issue = [&](uint16_t* sk, uint16_t* sv, int it) {
+    const int kb = it * KS + grp;
+    if (kb >= nkb) return;
+    dma_tile<kAlongRows, NW>(rk, sk + grp * TILE, kb * kBlk, a.k.s.row, wq, lane);
+    dma_tile<kDownCols, NW>(rv, sv + grp * TILE, kb * kBlk, a.v.s.row, wq, lane);
   };
 
   const float c = a.scale_log2;  // scores are kept raw; exp2 arguments are c * s - m
@@ -291,9 +301,11 @@ __global__ __launch_bounds__(kThreads, 4) void flash_fwd_kernel(FwdArgs a) {
   zero(o[0]);
   zero(o[1]);
 
-  auto compute = [&](const uint16_t* sk, const uint16_t* sv, int kb) {
-    const int k0 = kb * kBlk;
-    if (k0 >= kend_w) return;  // every query of this wave precedes the block
+  auto compute = [&](const uint16_t* skg, const uint16_t* svg, int it) {
+    const uint16_t* sk = skg + grp * TILE;
+    const uint16_t* sv = svg + grp * TILE;
+    const int k0 = (it * KS + grp) * kBlk;
+    if (k0 >= kend_w) return;  // every query of this wave precedes the block (or no such block)
     // S^T (keys x queries): lane (query, g) holds keys k0 + kt*32 + 8(r/4) + 4g + r%4
     f32x16 s[2];
 #pragma unroll
@@ -363,25 +375,53 @@ __global__ __launch_bounds__(kThreads, 4) void flash_fwd_kernel(FwdArgs a) {
       }
   };
 
-  if (nkb > 0) issue(sK0, sV0, 0);
-  for (int kb = 0; kb < nkb; kb += 2) {
+  issue(sK0, sV0, 0);
+  for (int it = 0; it < nit; it += 2) {
     wait_vm<0>();
     __syncthreads();
-    if (kb + 1 < nkb) issue(sK1, sV1, kb + 1);
-    compute(sK0, sV0, kb);
-    if (kb + 1 >= nkb) break;
+    issue(sK1, sV1, it + 1);
+    compute(sK0, sV0, it);
+    if (it + 1 >= nit) break;
     wait_vm<0>();
     __syncthreads();
-    if (kb + 2 < nkb) issue(sK0, sV0, kb + 2);
-    compute(sK1, sV1, kb + 1);
+    issue(sK0, sV0, it + 2);
+    compute(sK1, sV1, it + 1);
   }
 
-  const float lt = l + __shfl_xor(l, 32, kWave);
+  float lt = l + __shfl_xor(l, 32, kWave);
+  __syncthreads();  // every wave is done reading the K / V blocks
+  if constexpr (KS > 1) {
+    // group 1's (base, sum, O) merge into group 0's; a group that saw no key of
+    // a query has base -inf and weight 0
+    constexpr int PER = 32 * 64;  // floats of O per wave, in sV0; base and sum in sV1
+    static_assert(KS == 2 && NW * PER * 4 <= KS * TILE * 2, "a partial per wave of a group in one buffer");
+    float* const po = reinterpret_cast<float*>(sV0) + wq * PER;
+    float* const ps = reinterpret_cast<float*>(sV1) + wq * 128;
+    if (grp == 1) {
+      ps[lane] = m;
+      ps[64 + lane] = lt;
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) po[(dt * 16 + r) * 64 + lane] = o[dt][r];
+    }
+    __syncthreads();
+    if (grp == 1) return;
+    const float m2 = ps[lane], l2 = ps[64 + lane];
+    const float mn = fmaxf(m, m2);
+    const float c1 = m == -INFINITY ? 0.f : fast_exp2(m - mn), c2 = m2 == -INFINITY ? 0.f : fast_exp2(m2 - mn);
+    lt = lt * c1 + l2 * c2;
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[dt][r] = o[dt][r] * c1 + po[(dt * 16 + r) * 64 + lane] * c2;
+    m = mn;
+  }
   const float inv = qvalid ? 1.f / lt : 0.f;
   if (qvalid && g == 0) a.L[((int64_t)b * a.H + h) * S + q] = (m + fast_log2(lt)) * kLn2;
-  __syncthreads();  // every wave is done reading the K / V blocks
-  store_rows_staged(wave == 0 ? sK0 : wave == 1 ? sK1 : wave == 2 ? sV0 : sV1, o, inv, g, l32, lane, a.o, b, h, qw0,
-                    S);
+  // group 0's slabs: sK0 is free of partials
+  uint16_t* slab = KS > 1 ? sK0 + wave * 32 * kD : wave == 0 ? sK0 : wave == 1 ? sK1 : wave == 2 ? sV0 : sV1;
+  store_rows_staged(slab, o, inv, g, l32, lane, a.o, b, h, qw0, S);
 }
 
 // ---------------------------------------------------------------------------
@@ -392,6 +432,16 @@ struct PreArgs {
   Op o, dout;
   float* D;
 };
+// sum of the 8 products of two 16-byte chunks, in column order
+__device__ __forceinline__ float dot8(const u32x4& x, const u32x4& y) {
+  float acc = 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    acc = __builtin_fmaf(bf16_lo(x[j]), bf16_lo(y[j]), acc);
+    acc = __builtin_fmaf(bf16_hi(x[j]), bf16_hi(y[j]), acc);
+  }
+  return acc;
+}
 // grid (ceil(S / 32), H, B): 32 rows per workgroup, 8 lanes per row, 16 bytes
 // of O and of dO per lane; no division in the index math
 __global__ __launch_bounds__(256) void flash_bwd_pre_kernel(PreArgs a) {
@@ -402,8 +452,7 @@ __global__ __launch_bounds__(256) void flash_bwd_pre_kernel(PreArgs a) {
   if (s < a.S) {
     const u32x4 x = *reinterpret_cast<const u32x4*>(a.o.at(b, h, s) + part * 8);
     const u32x4 y = *reinterpret_cast<const u32x4*>(a.dout.at(b, h, s) + part * 8);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc += bf16_lo(x[j]) * bf16_lo(y[j]) + bf16_hi(x[j]) * bf16_hi(y[j]);
+    acc = dot8(x, y);
   }
   acc += __shfl_xor(acc, 1, kWave);
   acc += __shfl_xor(acc, 2, kWave);
@@ -417,6 +466,8 @@ struct BwdArgs {
   Op q, k, v, dout;
   const float* L;  // natural-log lse
   const float* D;
+  Op o;         // dQ forming D itself: O and where D goes
+  float* Dout;
   OutOp dq, dk, dv;
 };
 
@@ -426,22 +477,25 @@ struct BwdArgs {
 // along rows (S = Q K^T, dP = dO V^T) and down columns (dV += dO^T P,
 // dK += Q^T dS) from the one LDS copy.
 // ---------------------------------------------------------------------------
+template <int KS>
 __global__ __launch_bounds__(kThreads, 2) void flash_bwd_dkdv_kernel(BwdArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t sQ0[kBlk * kD];
-  __shared__ __attribute__((aligned(16))) uint16_t sQ1[kBlk * kD];
-  __shared__ __attribute__((aligned(16))) uint16_t sO0[kBlk * kD];
-  __shared__ __attribute__((aligned(16))) uint16_t sO1[kBlk * kD];
-  __shared__ __attribute__((aligned(16))) float sL0[kBlk];
-  __shared__ __attribute__((aligned(16))) float sL1[kBlk];
-  __shared__ __attribute__((aligned(16))) float sD0[kBlk];
-  __shared__ __attribute__((aligned(16))) float sD1[kBlk];
+  constexpr int ROWS = kRows / KS, NW = 4 / KS, TILE = kBlk * kD;
+  __shared__ __attribute__((aligned(16))) uint16_t sQ0[KS * TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t sQ1[KS * TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t sO0[KS * TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t sO1[KS * TILE];
+  __shared__ __attribute__((aligned(16))) float sL0[KS * kBlk];
+  __shared__ __attribute__((aligned(16))) float sL1[KS * kBlk];
+  __shared__ __attribute__((aligned(16))) float sD0[KS * kBlk];
+  __shared__ __attribute__((aligned(16))) float sD1[KS * kBlk];
   const int S = a.S;
   const TileCoord tc = tile_coord(a.H, a.B);
   const int kt_idx = tc.rank;  // low key tiles see the most queries: launched first
   const int h = tc.h, b = tc.b;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = KS == 1 ? 0 : wave / NW, wq = KS == 1 ? wave : wave % NW;  // query group, wave within it
   const int g = lane >> 5, l32 = lane & 31;
-  const int kw0 = kt_idx * kRows + wave * 32;
+  const int kw0 = kt_idx * ROWS + wq * 32;
   const int key = kw0 + l32;
   const bool kvalid = key < S;
   const int64_t lbase = ((int64_t)b * a.H + h) * S;
@@ -462,24 +516,33 @@ __global__ __launch_bounds__(kThreads, 2) void flash_bwd_dkdv_kernel(BwdArgs a) 
   zero(dv[0]);
   zero(dv[1]);
 
-  const int qstart = a.causal ? (kt_idx * kRows) / kBlk * kBlk : 0;
+  const int qstart = a.causal ? (kt_idx * ROWS) / kBlk * kBlk : 0;
   const int nqb = (S - qstart + kBlk - 1) / kBlk;
+  const int nit = (nqb + KS - 1) / KS;  // group grp takes blocks it * KS + grp
   const __amdgpu_buffer_rsrc_t rq = head_rsrc(a.q.at(b, h, 0), S, a.q.s.row);
   const __amdgpu_buffer_rsrc_t ro = head_rsrc(a.dout.at(b, h, 0), S, a.dout.s.row);
   const __amdgpu_buffer_rsrc_t rl = make_rsrc(a.L + lbase, (uint32_t)S * 4u);
   const __amdgpu_buffer_rsrc_t rd = make_rsrc(a.D + lbase, (uint32_t)S * 4u);
-  auto issue = [&](uint16_t* sq, uint16_t* so, float* sl, float* sd, int qb) {
+  auto issue = [&](uint16_t* sq, uint16_t* so, float* sl, float* sd, int it) {
+    const int qb = it * KS + grp;
+    if (qb >= nqb) return;
     const int q0 = qstart + qb * kBlk;
-    dma_tile(rq, sq, q0, a.q.s.row, wave, lane);
-    dma_tile(ro, so, q0, a.dout.s.row, wave, lane);
+    dma_tile<kBoth, NW>(rq, sq + grp * TILE, q0, a.q.s.row, wq, lane);
+    dma_tile<kBoth, NW>(ro, so + grp * TILE, q0, a.dout.s.row, wq, lane);
     if (lane < 16) {  // 64 floats of L (wave 0) and of D (wave 1); rows past S read zero
-      if (wave == 0) dma16(rl, sl, (uint32_t)(q0 + lane * 4) * 4u, 0);
-      if (wave == 1) dma16(rd, sd, (uint32_t)(q0 + lane * 4) * 4u, 0);
+      if (wq == 0) dma16(rl, sl + grp * kBlk, (uint32_t)(q0 + lane * 4) * 4u, 0);
+      if (wq == 1) dma16(rd, sd + grp * kBlk, (uint32_t)(q0 + lane * 4) * 4u, 0);
     }
   };
   const float c = a.scale_log2;
 
-  auto compute = [&](const uint16_t* sq, const uint16_t* so, const float* sl, const float* sd, int qb) {
+  auto compute = [&](const uint16_t* sqg, const uint16_t* sog, const float* slg, const float* sdg, int it) {
+    const int qb = it * KS + grp;
+    if (KS > 1 && qb >= nqb) return;
+    const uint16_t* sq = sqg + grp * TILE;
+    const uint16_t* so = sog + grp * TILE;
+    const float* sl = slg + grp * kBlk;
+    const float* sd = sdg + grp * kBlk;
     const int q0 = qstart + qb * kBlk;
     // this wave's keys see queries >= kw0 only (causal)
     if (a.causal && q0 + kBlk - 1 < kw0) return;
@@ -539,52 +602,86 @@ __global__ __launch_bounds__(kThreads, 2) void flash_bwd_dkdv_kernel(BwdArgs a) 
   // them in place as -L log2(e) and -D (one vector op each per block instead of
   // one per score in every wave).
   auto prep = [&](float* sl, float* sd) {
-    if (lane < 16 && wave < 2) {
-      float* p = (wave == 0 ? sl : sd) + lane * 4;
-      const float f = wave == 0 ? -kLog2e : -1.f;
+    if (lane < 16 && wq < 2) {
+      float* p = (wq == 0 ? sl : sd) + grp * kBlk + lane * 4;
+      const float f = wq == 0 ? -kLog2e : -1.f;
       f32x4 x = *reinterpret_cast<const f32x4*>(p);
 #pragma unroll
       for (int e = 0; e < 4; ++e) x[e] *= f;
       *reinterpret_cast<f32x4*>(p) = x;
     }
   };
-  if (nqb > 0) issue(sQ0, sO0, sL0, sD0, 0);
-  for (int qb = 0; qb < nqb; qb += 2) {
+  issue(sQ0, sO0, sL0, sD0, 0);
+  for (int it = 0; it < nit; it += 2) {
     wait_vm<0>();
     prep(sL0, sD0);
     __syncthreads();
-    if (qb + 1 < nqb) issue(sQ1, sO1, sL1, sD1, qb + 1);
-    compute(sQ0, sO0, sL0, sD0, qb);
-    if (qb + 1 >= nqb) break;
+    issue(sQ1, sO1, sL1, sD1, it + 1);
+    compute(sQ0, sO0, sL0, sD0, it);
+    if (it + 1 >= nit) break;
     wait_vm<0>();
     prep(sL1, sD1);
     __syncthreads();
-    if (qb + 2 < nqb) issue(sQ0, sO0, sL0, sD0, qb + 2);
-    compute(sQ1, sO1, sL1, sD1, qb + 1);
+    issue(sQ0, sO0, sL0, sD0, it + 2);
+    compute(sQ1, sO1, sL1, sD1, it + 1);
   }
   __syncthreads();  // every wave is done reading the Q / dO blocks
-  uint16_t* slab = wave == 0 ? sQ0 : wave == 1 ? sQ1 : wave == 2 ? sO0 : sO1;
-  store_rows_staged(slab, dk, a.scale, g, l32, lane, a.dk, b, h, kw0, S);
-  store_rows_staged(slab + 32 * kD, dv, 1.f, g, l32, lane, a.dv, b, h, kw0, S);
+  if constexpr (KS == 1) {
+    uint16_t* slab = wave == 0 ? sQ0 : wave == 1 ? sQ1 : wave == 2 ? sO0 : sO1;
+    store_rows_staged(slab, dk, a.scale, g, l32, lane, a.dk, b, h, kw0, S);
+    store_rows_staged(slab + 32 * kD, dv, 1.f, g, l32, lane, a.dv, b, h, kw0, S);
+  } else {
+    // group 0 finishes dK, group 1 dV: each leaves the other's partial (32 floats
+    // per lane, 8 KB per wave) and adds the one it is given
+    constexpr int PER = 32 * 64;
+    static_assert(KS == 2 && NW * PER * 4 <= KS * TILE * 2, "a partial per wave of a group in one buffer");
+    auto put = [&](float* p, const f32x16 (&v)[2]) {
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) p[(dt * 16 + r) * 64 + lane] = v[dt][r];
+    };
+    auto add = [&](f32x16 (&v)[2], const float* p) {
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[dt][r] += p[(dt * 16 + r) * 64 + lane];
+    };
+    float* pk = reinterpret_cast<float*>(sQ0) + wq * PER;  // dK of group 1
+    float* pv = reinterpret_cast<float*>(sO0) + wq * PER;  // dV of group 0
+    if (grp == 0) put(pv, dv);
+    else put(pk, dk);
+    __syncthreads();
+    if (grp == 0) {
+      add(dk, pk);
+      store_rows_staged(sQ1 + wq * 32 * kD, dk, a.scale, g, l32, lane, a.dk, b, h, kw0, S);
+    } else {
+      add(dv, pv);
+      store_rows_staged(sO1 + wq * 32 * kD, dv, 1.f, g, l32, lane, a.dv, b, h, kw0, S);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
 // dQ: workgroup = 128 queries, streams 64-key blocks up to the diagonal; the
 // K tile is read along rows (S) and down columns (dQ += dS K).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads, 3) void flash_bwd_dq_kernel(BwdArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t sK0[kBlk * kD];
-  __shared__ __attribute__((aligned(16))) uint16_t sK1[kBlk * kD];
-  __shared__ __attribute__((aligned(16))) uint16_t sV0[kBlk * kD];
-  __shared__ __attribute__((aligned(16))) uint16_t sV1[kBlk * kD];
+template <int KS, bool kFormD>
+__global__ __launch_bounds__(kThreads, KS == 1 ? 3 : 2) void flash_bwd_dq_kernel(BwdArgs a) {
+  constexpr int ROWS = kRows / KS, NW = 4 / KS, TILE = kBlk * kD;
+  __shared__ __attribute__((aligned(16))) uint16_t sK0[KS * TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t sK1[KS * TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t sV0[KS * TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t sV1[KS * TILE];
   const int S = a.S;
-  const int nqt = (S + kRows - 1) / kRows;
+  const int nqt = (S + ROWS - 1) / ROWS;
   const TileCoord tc = tile_coord(a.H, a.B);
   const int qt = nqt - 1 - tc.rank;
   const int h = tc.h, b = tc.b;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, l32 = lane & 31;
-  const int qw0 = qt * kRows + wave * 32;
+  const int grp = KS == 1 ? 0 : wave / NW, wq = KS == 1 ? wave : wave % NW;  // key group, wave within it
+  const int qw0 = qt * ROWS + wq * 32;
   const int q = qw0 + l32;
   const bool qvalid = q < S;
   const int64_t lbase = ((int64_t)b * a.H + h) * S;
@@ -601,24 +698,45 @@ __global__ __launch_bounds__(kThreads, 3) void flash_bwd_dq_kernel(BwdArgs a) {
   }
   const float c = a.scale_log2;
   const float nLq = qvalid ? -a.L[lbase + q] * kLog2e : -INFINITY;
-  const float Dq = qvalid ? a.D[lbase + q] : 0.f;
+  float Dq;
+  if constexpr (kFormD) {
+    // D = rowsum(dO o O): lane (q, g) holds chunks 2 ks + g of its dO row; the
+    // chunk sums combine in the preprocess kernel's order, bit for bit
+    const uint16_t* op = a.o.at(b, h, qvalid ? q : 0);
+    float c[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const u32x4 x = __builtin_bit_cast(u32x4, global_frag(op + ks * 16 + g * 8, qvalid));
+      c[ks] = dot8(x, __builtin_bit_cast(u32x4, df[ks]));
+      c[ks] += __shfl_xor(c[ks], 32, kWave);
+    }
+    Dq = (c[0] + c[1]) + (c[2] + c[3]);
+    if (qvalid && g == 0 && grp == 0) a.Dout[lbase + q] = Dq;
+  } else {
+    Dq = qvalid ? a.D[lbase + q] : 0.f;
+  }
 
-  const int kend_wg = a.causal ? min(S, qt * kRows + kRows) : S;
+  const int kend_wg = a.causal ? min(S, qt * ROWS + ROWS) : S;
   const int kend_w = a.causal ? min(S, qw0 + 32) : S;
   const int nkb = (kend_wg + kBlk - 1) / kBlk;
+  const int nit = (nkb + KS - 1) / KS;  // group grp takes blocks it * KS + grp
   const __amdgpu_buffer_rsrc_t rk = head_rsrc(a.k.at(b, h, 0), S, a.k.s.row);
   const __amdgpu_buffer_rsrc_t rv = head_rsrc(a.v.at(b, h, 0), S, a.v.s.row);
-  auto issue = [&](uint16_t* sk, uint16_t* sv, int kb) {
-    dma_tile(rk, sk, kb * kBlk, a.k.s.row, wave, lane);
-    dma_tile(rv, sv, kb * kBlk, a.v.s.row, wave, lane);
+  auto issue = [&](uint16_t* sk, uint16_t* sv, int it) {
+    const int kb = it * KS + grp;
+    if (kb >= nkb) return;
+    dma_tile<kBoth, NW>(rk, sk + grp * TILE, kb * kBlk, a.k.s.row, wq, lane);
+    dma_tile<kBoth, NW>(rv, sv + grp * TILE, kb * kBlk, a.v.s.row, wq, lane);
   };
 
   f32x16 dq[2];
   zero(dq[0]);
   zero(dq[1]);
 
-  auto compute = [&](const uint16_t* sk, const uint16_t* sv, int kb) {
-    const int k0 = kb * kBlk;
+  auto compute = [&](const uint16_t* skg, const uint16_t* svg, int it) {
+    const uint16_t* sk = skg + grp * TILE;
+    const uint16_t* sv = svg + grp * TILE;
+    const int k0 = (it * KS + grp) * kBlk;
     if (k0 >= kend_w) return;
     const bool need_mask = (a.causal && k0 + kBlk - 1 > qw0) || (k0 + kBlk > S);
 #pragma unroll
@@ -653,17 +771,36 @@ __global__ __launch_bounds__(kThreads, 3) void flash_bwd_dq_kernel(BwdArgs a) {
     }
   };
 
-  if (nkb > 0) issue(sK0, sV0, 0);
-  for (int kb = 0; kb < nkb; kb += 2) {
+  issue(sK0, sV0, 0);
+  for (int it = 0; it < nit; it += 2) {
     wait_vm<0>();
     __syncthreads();
-    if (kb + 1 < nkb) issue(sK1, sV1, kb + 1);
-    compute(sK0, sV0, kb);
-    if (kb + 1 >= nkb) break;
+    issue(sK1, sV1, it + 1);
+    compute(sK0, sV0, it);
+    if (it + 1 >= nit) break;
     wait_vm<0>();
     __syncthreads();
-    if (kb + 2 < nkb) issue(sK0, sV0, kb + 2);
-    compute(sK1, sV1, kb + 1);
+    issue(sK0, sV0, it + 2);
+    compute(sK1, sV1, it + 1);
+  }
+  if constexpr (KS > 1) {
+    // group 0 adds group 1's partial dQ
+    constexpr int PER = 32 * 64;  // floats per wave
+    static_assert(KS == 2 && NW * PER * 4 <= KS * TILE * 2, "a partial per wave of a group in one buffer");
+    __syncthreads();  // every wave is done reading the K / V blocks
+    float* p = reinterpret_cast<float*>(sK0) + wq * PER;
+    if (grp == 1) {
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) p[(dt * 16 + r) * 64 + lane] = dq[dt][r];
+    }
+    __syncthreads();
+    if (grp == 1) return;
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dq[dt][r] += p[(dt * 16 + r) * 64 + lane];
   }
   // Direct 8-byte stores (lane = row): measured faster here than staging
   // through LDS, which needs a barrier that makes the waves with less causal
@@ -693,6 +830,25 @@ int check_common(int B, int H, int S, int d, int causal) {
   if (d != kD) return nl_set_error(NL_EUNSUPPORTED, "flash: d_head must be 64");
   if (causal != 0 && causal != 1) return nl_set_error(NL_EINVAL, "flash: causal must be 0 or 1");
   if (H > 65535 || B > 65535) return nl_set_error(NL_EINVAL, "flash: batch and heads must be <= 65535");
+  return NL_OK;
+}
+// Wave groups per workgroup (KS) and the grid of 128 / KS-row tiles. Two groups
+// (64-row tiles, each group every other block of the streamed side) pay while
+// all their workgroups are resident at once: their LDS allows two per CU, so up
+// to 256 tiles of 128 rows. Measured, one group -> two (us; forward, backward):
+//   16 tiles (1 x 200 x 8 heads)   6.1 -> 5.2    18.5 -> 14.3
+//   112 (2 x 777 x 8)             12.8 -> 9.7    39.3 -> 25.5
+//   256 (8 x 512 x 8)             10.3 -> 8.6    30.3 -> 23.4
+//   256 (1 x 4096 x 8)            50.2 -> 36.4  155.2 -> 94.6
+//   512 (16 x 512 x 8)            13.0 -> 14.2   37.5 -> 43.7
+// Four groups of 32 rows (128 KB of LDS, one workgroup per CU) gained on two
+// only under 64 tiles, at most 10%: not kept.
+constexpr int64_t kTwoGroupTiles = 256;
+int tile_grid(int batch, int heads, int seq, dim3& grid, int& ks) {
+  auto wgs = [&](int k) { return (int64_t)((seq + kRows / k - 1) / (kRows / k)) * heads * batch; };
+  ks = wgs(1) <= kTwoGroupTiles ? 2 : 1;
+  if (wgs(ks) >= ((int64_t)1 << 31)) return nl_set_error(NL_EUNSUPPORTED, "flash: too many tiles");
+  grid = dim3((unsigned)wgs(ks));
   return NL_OK;
 }
 int check_op(const void* p, const nl_attn_stride& s, const char* name) {
@@ -738,9 +894,12 @@ extern "C" int nl_flash_attention_fwd(void* stream, int batch, int heads, int se
   a.L = L;
   a.H = heads;
   a.B = batch;
-  const int64_t wgs = (int64_t)((seq + kRows - 1) / kRows) * heads * batch;
-  if (wgs >= ((int64_t)1 << 31)) return nl_set_error(NL_EUNSUPPORTED, "flash: too many tiles");
-  hipLaunchKernelGGL(flash_fwd_kernel, dim3((unsigned)wgs), dim3(kThreads), 0, (hipStream_t)stream, a);
+  dim3 grid;
+  int ks;
+  NL_TRY(tile_grid(batch, heads, seq, grid, ks));
+  const hipStream_t st = (hipStream_t)stream;
+  if (ks == 2) hipLaunchKernelGGL(flash_fwd_kernel<2>, grid, dim3(kThreads), 0, st, a);
+  else hipLaunchKernelGGL(flash_fwd_kernel<1>, grid, dim3(kThreads), 0, st, a);
   return nl_check_launch("nl_flash_attention_fwd");
 }
 
@@ -786,13 +945,18 @@ static int fill_bwd(BwdArgs& a, int seq, int causal, float scale, const nl_bf16*
   return NL_OK;
 }
 
-static int bwd_grid(int batch, int heads, int seq, BwdArgs& a, dim3& grid) {
+// dQ; with Dout the kernel forms D itself and leaves it there (two wave groups only)
+static int launch_dq(void* stream, int batch, int heads, int seq, BwdArgs& a) {
   a.H = heads;
   a.B = batch;
-  const int64_t wgs = (int64_t)((seq + kRows - 1) / kRows) * heads * batch;
-  if (wgs >= ((int64_t)1 << 31)) return nl_set_error(NL_EUNSUPPORTED, "flash: too many tiles");
-  grid = dim3((unsigned)wgs);
-  return NL_OK;
+  dim3 grid;
+  int ks;
+  NL_TRY(tile_grid(batch, heads, seq, grid, ks));
+  const hipStream_t st = (hipStream_t)stream;
+  if (ks == 1) hipLaunchKernelGGL((flash_bwd_dq_kernel<1, false>), grid, dim3(kThreads), 0, st, a);
+  else if (a.Dout) hipLaunchKernelGGL((flash_bwd_dq_kernel<2, true>), grid, dim3(kThreads), 0, st, a);
+  else hipLaunchKernelGGL((flash_bwd_dq_kernel<2, false>), grid, dim3(kThreads), 0, st, a);
+  return nl_check_launch("nl_flash_attention_bwd_dq");
 }
 
 extern "C" int nl_flash_attention_bwd_dq(void* stream, int batch, int heads, int seq, int d_head, float scale,
@@ -802,14 +966,11 @@ extern "C" int nl_flash_attention_bwd_dq(void* stream, int batch, int heads, int
                                          nl_bf16* dQ, nl_attn_stride sdq) {
   NL_TRY(check_common(batch, heads, seq, d_head, causal));
   if (batch == 0 || heads == 0 || seq == 0) return NL_OK;
-  BwdArgs a;
+  BwdArgs a{};
   NL_TRY(fill_bwd(a, seq, causal, scale, Q, sq, K, sk, V, sv, dO, sdo, L, D));
   NL_TRY(check_op(dQ, sdq, "dQ"));
   a.dq = OutOp{dQ, sdq};
-  dim3 grid;
-  NL_TRY(bwd_grid(batch, heads, seq, a, grid));
-  hipLaunchKernelGGL(flash_bwd_dq_kernel, grid, dim3(kThreads), 0, (hipStream_t)stream, a);
-  return nl_check_launch("nl_flash_attention_bwd_dq");
+  return launch_dq(stream, batch, heads, seq, a);
 }
 
 extern "C" int nl_flash_attention_bwd_dkdv(void* stream, int batch, int heads, int seq, int d_head, float scale,
@@ -819,15 +980,20 @@ extern "C" int nl_flash_attention_bwd_dkdv(void* stream, int batch, int heads, i
                                            nl_bf16* dK, nl_attn_stride sdk, nl_bf16* dV, nl_attn_stride sdv) {
   NL_TRY(check_common(batch, heads, seq, d_head, causal));
   if (batch == 0 || heads == 0 || seq == 0) return NL_OK;
-  BwdArgs a;
+  BwdArgs a{};
   NL_TRY(fill_bwd(a, seq, causal, scale, Q, sq, K, sk, V, sv, dO, sdo, L, D));
   NL_TRY(check_op(dK, sdk, "dK"));
   NL_TRY(check_op(dV, sdv, "dV"));
   a.dk = OutOp{dK, sdk};
   a.dv = OutOp{dV, sdv};
+  a.H = heads;
+  a.B = batch;
   dim3 grid;
-  NL_TRY(bwd_grid(batch, heads, seq, a, grid));
-  hipLaunchKernelGGL(flash_bwd_dkdv_kernel, grid, dim3(kThreads), 0, (hipStream_t)stream, a);
+  int ks;
+  NL_TRY(tile_grid(batch, heads, seq, grid, ks));
+  const hipStream_t st = (hipStream_t)stream;
+  if (ks == 2) hipLaunchKernelGGL(flash_bwd_dkdv_kernel<2>, grid, dim3(kThreads), 0, st, a);
+  else hipLaunchKernelGGL(flash_bwd_dkdv_kernel<1>, grid, dim3(kThreads), 0, st, a);
   return nl_check_launch("nl_flash_attention_bwd_dkdv");
 }
 
@@ -847,12 +1013,32 @@ extern "C" int nl_flash_attention_bwd(void* stream, int batch, int heads, int se
   if (!ws) return nl_set_error(NL_EINVAL, "flash: null workspace");
   if (((uintptr_t)ws & 15) != 0) return nl_set_error(NL_EALIGN, "flash: workspace not 16-byte aligned");
   float* D = static_cast<float*>(ws);
-  NL_TRY(nl_flash_attention_bwd_preprocess(stream, batch, heads, seq, d_head, O, so, dO, sdo, D));
-  NL_TRY(nl_flash_attention_bwd_dkdv(stream, batch, heads, seq, d_head, scale, causal, Q, sq, K, sk, V, sv, dO, sdo,
-                                     L, D, dK, sdk, dV, sdv));
-  NL_TRY(nl_flash_attention_bwd_dq(stream, batch, heads, seq, d_head, scale, causal, Q, sq, K, sk, V, sv, dO, sdo,
-                                   L, D, dQ, sdq));
-  return NL_OK;
+  NL_TRY(check_op(O, so, "O"));
+  NL_TRY(check_op(dK, sdk, "dK"));
+  NL_TRY(check_op(dV, sdv, "dV"));
+  BwdArgs a{};
+  NL_TRY(fill_bwd(a, seq, causal, scale, Q, sq, K, sk, V, sv, dO, sdo, L, D));
+  NL_TRY(check_op(dQ, sdq, "dQ"));
+  a.dq = OutOp{dQ, sdq};
+  dim3 grid;
+  int ks;
+  NL_TRY(tile_grid(batch, heads, seq, grid, ks));
+  // With two wave groups dQ goes first and forms D on the way, which dK/dV then
+  // reads: the preprocess launch (4 us) is a tenth of such a backward. On a full
+  // chip D's O rows would only lengthen the start of every dQ workgroup: at 32 x
+  // 512 x 8 heads forward + backward took 100.0 us against 97.6 with the
+  // preprocess (at 4 x 4096, 349 against 350).
+  if (ks == 1) {
+    NL_TRY(nl_flash_attention_bwd_preprocess(stream, batch, heads, seq, d_head, O, so, dO, sdo, D));
+    NL_TRY(nl_flash_attention_bwd_dkdv(stream, batch, heads, seq, d_head, scale, causal, Q, sq, K, sk, V, sv, dO, sdo,
+                                       L, D, dK, sdk, dV, sdv));
+    return launch_dq(stream, batch, heads, seq, a);
+  }
+  a.o = Op{O, so};
+  a.Dout = D;
+  NL_TRY(launch_dq(stream, batch, heads, seq, a));
+  return nl_flash_attention_bwd_dkdv(stream, batch, heads, seq, d_head, scale, causal, Q, sq, K, sk, V, sv, dO, sdo,
+                                     L, D, dK, sdk, dV, sdv);
 }
 
 // ---------------------------------------------------------------------------

@@ -49,25 +49,6 @@ def prepare(device=None) -> None:
     _side_stream(dev, 1)
 
 
-def split(first, second, *keep) -> None:
-    """Run ``first()`` on the current stream and ``second()`` (which must not
-    allocate) on the op-internal side stream, concurrently when overlapping is
-    active, and join before returning: the current stream then waits for
-    both. ``keep``: every tensor ``second`` touches (referenced until here)."""
-    if _active is None:
-        first()
-        second()
-        return
-    main = torch.cuda.current_stream()
-    aux = _side_stream(_active["dev"], 1)
-    aux.wait_stream(main)
-    with torch.cuda.stream(aux):
-        second()
-    first()
-    main.wait_stream(aux)
-    del keep
-
-
 def active() -> bool:
     return _active is not None
 

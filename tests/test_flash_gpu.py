@@ -83,6 +83,36 @@ def test_flash_ragged_sequences(dev, B, H, S, causal):
     _check_against_oracle((O, L, dq, dk, dv), f32, B, H, S, causal)
 
 
+@pytest.mark.parametrize("B,H,S", [(2, 128, 33), (257, 1, 65), (52, 5, 97), (43, 3, 257)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_flash_tile_counts_on_both_sides(dev, B, H, S, causal):
+    """Ragged sequences at 256 tiles of 128 rows (two wave groups per
+    workgroup) and just above (one), and the backward's parts against the
+    whole: D formed inside the dQ kernel, dQ, dK and dV equal those of the
+    preprocess, dK/dV and dQ entry points bit for bit."""
+    import torch
+    from nlearn_amd import _lib
+    from nlearn_amd.attention import _stride4, flash_bwd_raw4, flash_fwd_raw4
+
+    (q, k, v, do), f32 = _rand_case(dev, B, H, S, seed=B + H + S)
+    O, L = flash_fwd_raw4(q, k, v, causal=causal)
+    dq, dk, dv = flash_bwd_raw4(q, k, v, O, do, L, causal=causal)
+    D = torch.full((B, H, S), float("nan"), dtype=torch.float32, device=dev)
+    parts = [torch.full_like(q, float("nan")) for _ in range(3)]
+    st = torch.cuda.current_stream(dev).cuda_stream
+    _lib.call("nl_flash_attention_bwd_preprocess", st, B, H, S, 64, O.data_ptr(), _stride4(O), do.data_ptr(),
+              _stride4(do), D.data_ptr())
+    ins = (0.125, int(causal), q.data_ptr(), _stride4(q), k.data_ptr(), _stride4(k), v.data_ptr(), _stride4(v),
+           do.data_ptr(), _stride4(do), L.data_ptr(), D.data_ptr())
+    _lib.call("nl_flash_attention_bwd_dkdv", st, B, H, S, 64, *ins, parts[1].data_ptr(), _stride4(parts[1]),
+              parts[2].data_ptr(), _stride4(parts[2]))
+    _lib.call("nl_flash_attention_bwd_dq", st, B, H, S, 64, *ins, parts[0].data_ptr(), _stride4(parts[0]))
+    torch.cuda.synchronize()
+    for whole, part in zip((dq, dk, dv), parts):
+        assert torch.equal(whole, part)
+    _check_against_oracle((O, L, dq, dk, dv), f32, B, H, S, causal)
+
+
 @pytest.mark.parametrize("B,H,S", [(1, 2, 545), (2, 1, 1024)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_flash_scores_growing_along_the_keys(dev, B, H, S, causal):
