@@ -88,10 +88,24 @@ __device__ __forceinline__ float wave_max(float v) {
   for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
   return v;
 }
+// The sum needs no LDS permute: lane exchanges within 16 lanes are DPP operands
+// of the add (once the lanes of a group agree, a mirror is as good as an xor),
+// and the two across rows are gfx950 row swaps.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
+  v += dpp<0xB1>(v);   // quad_perm 1,0,3,2
+  v += dpp<0x4E>(v);   // quad_perm 2,3,0,1
+  v += dpp<0x141>(v);  // row_half_mirror
+  v += dpp<0x140>(v);  // row_mirror
+  const uint32_t a = __float_as_uint(v);
+  const auto r16 = __builtin_amdgcn_permlane16_swap(a, a, false, false);
+  v = __uint_as_float(r16[0]) + __uint_as_float(r16[1]);
+  const uint32_t b = __float_as_uint(v);
+  const auto r32 = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return __uint_as_float(r32[0]) + __uint_as_float(r32[1]);
 }
 
 // ---------------------------------------------------------------------------

@@ -24,7 +24,7 @@ namespace {
 
 constexpr int kRowsPerBlock = 4;   // LayerNorm: one wave per row, 4 waves per workgroup
 constexpr int kMaxD = 4096;        // LayerNorm width limit (8 vectors of 8 per lane)
-constexpr int kLnBwdBlocks = 1024; // LayerNorm backward: partial rows of dgamma / dbeta
+constexpr int kLnBwdBlocks = 1024; // LayerNorm backward: partial rows of dgamma / dbeta the workspace holds
 constexpr int kColsumRows = 64;    // column sums: rows per partial
 
 // Lane `lane` holds columns (i*64 + lane)*8 .. +7 of the row in vector i.
@@ -57,11 +57,12 @@ __device__ __forceinline__ void load8f(const float* p, float f[8]) {
 
 // y = LN(s), s = x (+ r). With r, s is rounded to bf16 and stored to s_out (the
 // residual stream the next block reads) before it is normalised.
-// Rows per wave: short rows (D <= 1024) are handled several per wave, every
-// row's loads issued before the first is used, gamma and beta loaded once.
-template <int VPL>
-constexpr int ln_fwd_rows_per_wave() { return VPL == 1 ? 4 : VPL == 2 ? 2 : 1; }
-
+// One row per wave, every load (x, r, gamma, beta) issued before the first use.
+// Bound by HBM from about 8000 rows of 512 (16384: 67 MB in 15 us); below, by
+// the chain load -> sum -> squares -> store, which is why a wave takes one row
+// and sums without LDS permutes. Four rows per wave one after the other, with
+// permutes: 200 x 512 5.0 us against 2.4, 4096 x 512 7.3 against 5.4, 32768 x 512
+// 28.4 against 25.5.
 template <int VPL>
 __global__ __launch_bounds__(64 * kRowsPerBlock) void ln_fwd_kernel(int rows, int D, const uint16_t* __restrict__ x,
                                                                     const uint16_t* __restrict__ r,
@@ -70,21 +71,13 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void ln_fwd_kernel(int rows, in
                                                                     const float* __restrict__ beta,
                                                                     uint16_t* __restrict__ y, float* __restrict__ mean_out,
                                                                     float* __restrict__ rstd_out, float eps) {
-  constexpr int RPW = ln_fwd_rows_per_wave<VPL>();
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int row0 = blockIdx.x * kRowsPerBlock * RPW + wave;  // rows row0 + k * kRowsPerBlock
-  if (row0 >= rows) return;
-  // every load of the wave's rows (x, r) and of gamma, beta is issued before the first use
-  u32x4 xv[RPW][VPL], rv[RPW][VPL];
-#pragma unroll
-  for (int k = 0; k < RPW; ++k) {
-    const int row = row0 + k * kRowsPerBlock;
-    if (row < rows) {
-      load_row<VPL>(xv[k], x + (int64_t)row * D, D, lane);
-      if (r) load_row<VPL>(rv[k], r + (int64_t)row * D, D, lane);
-    }
-  }
+  const int row = blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int64_t off = (int64_t)row * D;
+  u32x4 xv[VPL], rv[VPL];
+  load_row<VPL>(xv, x + off, D, lane);
+  if (r) load_row<VPL>(rv, r + off, D, lane);
   float gg[VPL][8], bb[VPL][8];
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
@@ -94,56 +87,50 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void ln_fwd_kernel(int rows, in
       load8f(beta + c, bb[i]);
     }
   }
+  float f[VPL][8];
 #pragma unroll
-  for (int k = 0; k < RPW; ++k) {
-    const int row = row0 + k * kRowsPerBlock;
-    if (row >= rows) break;
-    const int64_t off = (int64_t)row * D;
-    float f[VPL][8];
-#pragma unroll
-    for (int i = 0; i < VPL; ++i) unpack8(xv[k][i], f[i]);
-    if (r) {
-#pragma unroll
-      for (int i = 0; i < VPL; ++i) {
-        float g[8];
-        unpack8(rv[k][i], g);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) f[i][j] = bf16_to_f32(f32_to_bf16(f[i][j] + g[j]));
-        const int c = (i * 64 + lane) * 8;
-        if (c < D) *reinterpret_cast<u32x4*>(s_out + off + c) = pack8(f[i]);
-      }
-    }
-    // columns beyond D hold zeros, so they add nothing to the sum
-    float s = 0.f;
-#pragma unroll
-    for (int i = 0; i < VPL; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) s += f[i][j];
-    const float mean = wave_sum(s) / (float)D;
-    float v = 0.f;
+  for (int i = 0; i < VPL; ++i) unpack8(xv[i], f[i]);
+  if (r) {
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-      const bool in = (i * 64 + lane) * 8 < D;
+      float g[8];
+      unpack8(rv[i], g);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float d = in ? f[i][j] - mean : 0.f;
-        v += d * d;
-      }
-    }
-    const float rstd = rsqrtf(wave_sum(v) / (float)D + eps);
-#pragma unroll
-    for (int i = 0; i < VPL; ++i) {
+      for (int j = 0; j < 8; ++j) f[i][j] = bf16_to_f32(f32_to_bf16(f[i][j] + g[j]));
       const int c = (i * 64 + lane) * 8;
-      if (c >= D) continue;
-      float o[8];
+      if (c < D) *reinterpret_cast<u32x4*>(s_out + off + c) = pack8(f[i]);
+    }
+  }
+  // columns beyond D hold zeros, so they add nothing to the sum
+  float s = 0.f;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = (f[i][j] - mean) * rstd * gg[i][j] + bb[i][j];
-      *reinterpret_cast<u32x4*>(y + off + c) = pack8(o);
+  for (int i = 0; i < VPL; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s += f[i][j];
+  const float mean = wave_sum(s) / (float)D;
+  float v = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPL; ++i) {
+    const bool in = (i * 64 + lane) * 8 < D;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float d = in ? f[i][j] - mean : 0.f;
+      v += d * d;
     }
-    if (lane == 0) {
-      mean_out[row] = mean;
-      rstd_out[row] = rstd;
-    }
+  }
+  const float rstd = rsqrtf(wave_sum(v) / (float)D + eps);
+#pragma unroll
+  for (int i = 0; i < VPL; ++i) {
+    const int c = (i * 64 + lane) * 8;
+    if (c >= D) continue;
+    float o[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = (f[i][j] - mean) * rstd * gg[i][j] + bb[i][j];
+    *reinterpret_cast<u32x4*>(y + off + c) = pack8(o);
+  }
+  if (lane == 0) {
+    mean_out[row] = mean;
+    rstd_out[row] = rstd;
   }
 }
 
@@ -153,7 +140,7 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void ln_fwd_kernel(int rows, in
 // columns [4q, 4q+4) of its strip; the 64 phase sums are then added in groups
 // of 4 (phases 4g..4g+3) and the 16 group sums in g order. The strips are
 // narrow so that a 512-column sum still spreads over 32 workgroups per pair
-// with every row load in flight at once (P <= 1024: 16 loads a thread).
+// with every row load in flight at once (P <= 512: 8 loads a thread).
 __device__ __forceinline__ void sum_partials_strip(int bx, int pair, int P, int D, const float* __restrict__ part0,
                                                    float* __restrict__ out0, const float* __restrict__ part1,
                                                    float* __restrict__ out1, int accumulate) {
@@ -224,8 +211,10 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void ln_bwd_kernel(
                        prev.dbeta, prev.accumulate);
     return;
   }
-  __shared__ float sg[VPL * 512];
-  __shared__ float sb[VPL * 512];
+  // [wave][j][lane]: the sums of column (i*64 + lane)*8 + j; the 72-float pitch
+  // keeps both the per-wave writes and the per-column reads off shared banks
+  __shared__ float sg[kRowsPerBlock][8 * 72];
+  __shared__ float sb[kRowsPerBlock][8 * 72];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   float ag[VPL][8], ab[VPL][8], gam[VPL][8];
@@ -302,22 +291,22 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void ln_bwd_kernel(
     row = nxt;
   }
   // combine the 4 waves in wave order (deterministic), one partial row per workgroup
-  for (int w = 0; w < kRowsPerBlock; ++w) {
-    if (wave == w) {
 #pragma unroll
-      for (int i = 0; i < VPL; ++i)
+  for (int i = 0; i < VPL; ++i) {
+    if (i > 0) __syncthreads();
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int c = (i * 64 + lane) * 8 + j;
-          sg[c] = (w == 0 ? 0.f : sg[c]) + ag[i][j];
-          sb[c] = (w == 0 ? 0.f : sb[c]) + ab[i][j];
-        }
+    for (int j = 0; j < 8; ++j) {
+      sg[wave][j * 72 + lane] = ag[i][j];
+      sb[wave][j * 72 + lane] = ab[i][j];
     }
     __syncthreads();
-  }
-  for (int c = threadIdx.x; c < D; c += blockDim.x) {
-    part_g[(int64_t)blockIdx.x * D + c] = sg[c];
-    part_b[(int64_t)blockIdx.x * D + c] = sb[c];
+    for (int e = threadIdx.x; e < 512; e += blockDim.x) {
+      const int c = i * 512 + e;
+      if (c >= D) break;
+      const int o = (e & 7) * 72 + (e >> 3);
+      part_g[(int64_t)blockIdx.x * D + c] = ((sg[0][o] + sg[1][o]) + sg[2][o]) + sg[3][o];
+      part_b[(int64_t)blockIdx.x * D + c] = ((sb[0][o] + sb[1][o]) + sb[2][o]) + sb[3][o];
+    }
   }
 }
 
@@ -716,7 +705,15 @@ int vectors_per_lane(int D) {
   return v <= 1 ? 1 : v <= 2 ? 2 : v <= 4 ? 4 : 8;
 }
 
-int ln_bwd_blocks(int rows) { return std::min(kLnBwdBlocks, (rows + kRowsPerBlock - 1) / kRowsPerBlock); }
+// Workgroups of the LayerNorm backward, each leaving one partial row of dgamma
+// and dbeta: few, because the partials cost as much traffic per workgroup as
+// 8 rows of data and their sum is a launch that waits for all of them; enough
+// to keep the loads in flight. Measured with the sum (us, 1024 / 512 / 256):
+//   4096 x 512   15.1 / 11.6 / 10.3     16384 x 512   24.0 / 21.3 / 26.1
+//   8192 x 512   18.4 / 14.7 / 16.0     32768 x 512   35.9 / 32.2 / 43.0
+int ln_bwd_blocks(int rows) {
+  return std::min(rows >= 8192 ? 512 : 256, (rows + kRowsPerBlock - 1) / kRowsPerBlock);
+}
 
 }  // namespace
 }  // namespace nl
@@ -736,14 +733,13 @@ extern "C" int nl_layernorm_fwd(void* stream, int rows, int D, const nl_bf16* x,
     return nl_set_error(NL_EALIGN, "layernorm: buffers must be 16-byte aligned");
   const dim3 block(64 * kRowsPerBlock);
   hipStream_t st = (hipStream_t)stream;
+  const dim3 grid((rows + kRowsPerBlock - 1) / kRowsPerBlock);
   switch (vectors_per_lane(D)) {
 #define NL_LNF(N)                                                                                                    \
-  case N: {                                                                                                          \
-    const int per = kRowsPerBlock * ln_fwd_rows_per_wave<N>();                                                       \
-    hipLaunchKernelGGL(ln_fwd_kernel<N>, dim3((rows + per - 1) / per), block, 0, st, rows, D, x, residual, sum_out,  \
-                       gamma, beta, y, mean, rstd, eps);                                                             \
-    break;                                                                                                           \
-  }
+  case N:                                                                                                            \
+    hipLaunchKernelGGL(ln_fwd_kernel<N>, grid, block, 0, st, rows, D, x, residual, sum_out, gamma, beta, y, mean,    \
+                       rstd, eps);                                                                                   \
+    break;
     NL_LNF(1)
     NL_LNF(2)
     NL_LNF(4)
@@ -755,7 +751,7 @@ extern "C" int nl_layernorm_fwd(void* stream, int rows, int D, const nl_bf16* x,
 
 extern "C" size_t nl_layernorm_bwd_ws_bytes(int rows, int D) {
   if (rows <= 0 || D <= 0) return 0;
-  return (size_t)2 * ln_bwd_blocks(rows) * D * sizeof(float);
+  return (size_t)2 * std::min(kLnBwdBlocks, (rows + kRowsPerBlock - 1) / kRowsPerBlock) * D * sizeof(float);
 }
 
 #define NL_TRY(x)        \

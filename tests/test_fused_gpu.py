@@ -86,6 +86,13 @@ def test_layernorm_fwd_bwd(dev, rows, D, residual):
         assert torch.equal(a, c)                           # fixed reduction order
 
 
+@pytest.mark.parametrize("rows,D", [(1023, 512), (1026, 512), (8191, 256), (8193, 264)])
+def test_layernorm_around_the_workgroup_limits(dev, rows, D):
+    """Row counts around the backward's two workgroup limits (256 up to 8191
+    rows, 512 above), where waves take unequal numbers of rows."""
+    test_layernorm_fwd_bwd(dev, rows, D, True)
+
+
 def test_layernorm_autograd_chain(dev):
     """add_layer_norm: gradients w.r.t. x and r are equal and include the LN path."""
     import torch
