@@ -55,7 +55,7 @@ def _prep(t: torch.Tensor) -> torch.Tensor:
 
 
 def _stream(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _lib.stream_of(t)
 
 
 def _new_bshd(B, H, S, D, device):
@@ -119,17 +119,33 @@ def flash_attention(q, k, v, causal: bool = True, scale: float | None = None):
 
 
 class _FlashQKV(torch.autograd.Function):
-    """Attention straight from the fused projection output qkv (B, S, 3, H, D)."""
+    """Attention straight from the fused projection output qkv (B, S, 3, H, D)
+    (contiguous bf16: flash_attention_qkv sees to it)."""
 
     @staticmethod
     def forward(ctx, qkv, causal, scale):
         B, S, three, H, D = qkv.shape
         assert three == 3
-        q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
-        O, L = flash_fwd_raw4(q, k, v, causal, scale)
+        if qkv.data_ptr() % 16 or D % 8 or D < 64 or not qkv.numel():
+            q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
+            O, L = flash_fwd_raw4(q, k, v, causal, scale)
+            out = O.permute(0, 2, 1, 3).reshape(B, S, H * D)  # storage is already (B, S, H, D)
+        else:
+            # the same call on the layout itself, without building the six views
+            _check_device(qkv)
+            O = _new_bshd(B, H, S, D, qkv.device)
+            out = O.permute(0, 2, 1, 3).view(B, S, H * D)
+            L = torch.empty((B, H, S), dtype=torch.float32, device=qkv.device)
+            row = H * D
+            s3 = _lib.AttnStride(3 * S * row, D, 3 * row)
+            p = qkv.data_ptr()
+            _lib.call("nl_flash_attention_fwd", _stream(qkv), B, H, S, D,
+                      1.0 / math.sqrt(D) if scale is None else float(scale), int(bool(causal)),
+                      p, s3, p + 2 * row, s3, p + 4 * row, s3, O.data_ptr(), _lib.AttnStride(S * row, D, row),
+                      L.data_ptr())
         ctx.save_for_backward(qkv, O, L)
         ctx.causal, ctx.scale = causal, scale
-        return O.permute(0, 2, 1, 3).reshape(B, S, H * D)  # storage is already (B, S, H, D)
+        return out
 
     @staticmethod
     def backward(ctx, dO):

@@ -57,7 +57,7 @@ def _targets(targets: torch.Tensor) -> torch.Tensor:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _lib.stream_of(t)
 
 
 def _ce_fwd_raw(logits: torch.Tensor, targets: torch.Tensor):

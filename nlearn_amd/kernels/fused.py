@@ -30,7 +30,7 @@ _F32 = torch.float32
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _lib.stream_of(t)
 
 
 def _rows(x: torch.Tensor) -> torch.Tensor:
@@ -47,7 +47,7 @@ def _param(p: torch.Tensor) -> torch.Tensor:
     p = p.detach()
     if p.dtype != _F32:
         p = p.to(_F32)
-    return p.contiguous()
+    return p if p.is_contiguous() else p.contiguous()
 
 
 # ---------------------------------------------------------------------------

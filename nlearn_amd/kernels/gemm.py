@@ -71,6 +71,19 @@ def _kernel_ready(t: torch.Tensor) -> torch.Tensor:
     return view
 
 
+def _ready_ld(t: torch.Tensor):
+    """(_kernel_ready(t), its leading dimension), looked up once for the usual
+    operand that is ready as it is."""
+    if t.dtype is _BF16 and t.dim() == 2:
+        (rows, cols), (s0, s1) = t.shape, t.stride()
+        if (s1 == 1 or cols <= 1) and (rows <= 1 or s0 >= cols) and t.data_ptr() % 16 == 0:
+            ld = s0 if rows > 1 else (cols + 7) // 8 * 8
+            if ld % 8 == 0:
+                return t, ld
+    t = _kernel_ready(t)
+    return t, _ld(t)
+
+
 def padded_empty(rows: int, cols: int, dtype=_BF16, device="cuda") -> torch.Tensor:
     """A [rows, cols] view whose rows start on 16-byte boundaries (ld rounded to 8).
 
@@ -86,7 +99,8 @@ def padded_empty(rows: int, cols: int, dtype=_BF16, device="cuda") -> torch.Tens
     ld = (cols + 7) // 8 * 8 if cols < 1024 else (cols + 63) // 64 * 64
     if ld >= 1024 and ld % 1024 == 0:
         ld += 64
-    return torch.empty((rows, ld), dtype=dtype, device=device)[:, :cols]
+    t = torch.empty((rows, ld), dtype=dtype, device=device)
+    return t if ld == cols else t[:, :cols]
 
 
 EPI_NONE, EPI_BIAS, EPI_BIAS_GELU, EPI_DGELU = 0, 1, 2, 3
@@ -104,12 +118,10 @@ def gemm_raw(A: torch.Tensor, B: torch.Tensor, opA: str = "N", opB: str = "N", o
     ws: split-K workspace of at least ``gemm_ws_bytes`` bytes (allocated here if None).
     """
     _check_device(A, B)
-    A = _kernel_ready(A)
-    B = _kernel_ready(B)
-    M = A.shape[1] if opA == "T" else A.shape[0]
-    K = A.shape[0] if opA == "T" else A.shape[1]
-    Kb = B.shape[1] if opB == "T" else B.shape[0]
-    N = B.shape[0] if opB == "T" else B.shape[1]
+    A, lda = _ready_ld(A)
+    B, ldb = _ready_ld(B)
+    K, M = A.shape if opA == "T" else reversed(A.shape)
+    N, Kb = B.shape if opB == "T" else reversed(B.shape)
     if K != Kb:
         raise ValueError(f"gemm: inner dimensions differ ({K} vs {Kb})")
     if out is None:
@@ -118,7 +130,7 @@ def gemm_raw(A: torch.Tensor, B: torch.Tensor, opA: str = "N", opB: str = "N", o
         out = padded_empty(M, N, out_dtype, A.device)
     if out.dtype not in (_F32, _BF16):
         raise ValueError("gemm: output must be float32 or bfloat16")
-    if tuple(out.shape) != (M, N):
+    if out.shape != (M, N):
         raise ValueError(f"gemm: output shape {tuple(out.shape)} != {(M, N)}")
     if alpha_dev is not None and (alpha_dev.dtype != _F32 or not alpha_dev.is_cuda):
         raise ValueError("gemm: alpha_dev must be a float32 device scalar")
@@ -128,7 +140,7 @@ def gemm_raw(A: torch.Tensor, B: torch.Tensor, opA: str = "N", opB: str = "N", o
     if epi in (EPI_BIAS_GELU, EPI_DGELU):
         if aux is None or aux.dtype != _BF16 or tuple(aux.shape) != (M, N):
             raise ValueError(f"gemm: the GELU epilogues need a bf16 aux of shape {(M, N)}")
-    stream = torch.cuda.current_stream(A.device).cuda_stream
+    stream = _lib.stream_of(A)
     oa = _lib.NL_OP_T if opA == "T" else _lib.NL_OP_N
     ob = _lib.NL_OP_T if opB == "T" else _lib.NL_OP_N
     wsb = int(_lib.load().nl_gemm_ws_bytes(oa, ob, M, N, K))
@@ -137,7 +149,7 @@ def gemm_raw(A: torch.Tensor, B: torch.Tensor, opA: str = "N", opB: str = "N", o
     elif ws.numel() * ws.element_size() < wsb:
         raise ValueError("gemm: workspace too small")
     _lib.call("nl_gemm_fused", stream, oa, ob, M, N, K, float(alpha),
-              A.data_ptr(), _ld(A), B.data_ptr(), _ld(B), float(beta), out.data_ptr(),
+              A.data_ptr(), lda, B.data_ptr(), ldb, float(beta), out.data_ptr(),
               _lib.NL_DTYPE_F32 if out.dtype == _F32 else _lib.NL_DTYPE_BF16, _ld(out),
               alpha_dev.data_ptr() if alpha_dev is not None else None, int(epi),
               bias.data_ptr() if bias is not None else None,

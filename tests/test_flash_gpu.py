@@ -172,6 +172,42 @@ def test_flash_fused_qkv_layout_and_autograd(dev):
         assert rel_l2(got, ref) <= TOL
 
 
+def test_flash_qkv_direct_layout_equals_views(dev):
+    """The fused projection's layout handed to the kernel as it is against the
+    same values on an 8-byte boundary (copied through the strided views): the
+    outputs and gradients agree bit for bit, and neither keeps its memory once
+    the results are dropped (no cycle through the saved output)."""
+    import gc
+
+    import torch
+    from nlearn_amd.attention import flash_attention_qkv
+
+    B, S, H = 2, 70, 3
+    gen = torch.Generator(device=dev).manual_seed(3)
+    x = torch.randn((B, S, 3, H, 64), generator=gen, device=dev).to(torch.bfloat16)
+    off = torch.empty(x.numel() + 4, dtype=torch.bfloat16, device=dev)[4:].view(x.shape)
+    off.copy_(x)
+    assert x.data_ptr() % 16 == 0 and off.data_ptr() % 16 == 8
+    dO = torch.randn((B, S, H * 64), generator=gen, device=dev).to(torch.bfloat16)
+
+    def run(t):
+        t = t.detach().requires_grad_(True)
+        o = flash_attention_qkv(t)
+        return o.detach().clone(), torch.autograd.grad(o, t, dO)[0]
+
+    gc.collect()
+    gc.disable()
+    try:
+        (oa, ga), (ob, gb) = run(x), run(off)
+        before = torch.cuda.memory_allocated(dev)
+        for t in (x, off, x, off):
+            run(t)
+        assert torch.cuda.memory_allocated(dev) == before
+    finally:
+        gc.enable()
+    assert torch.equal(oa, ob) and torch.equal(ga, gb)
+
+
 def test_flash_reference_api_autograd(dev):
     import torch
     from nlearn_amd.attention import attention

@@ -175,3 +175,15 @@ def test_lm_head_chunk_bounds():
         for n in (1, 2, 3, 7):
             b = chunk_bounds(M, n)
             assert b[0] == 0 and b[-1] == M and all(x <= y for x, y in zip(b, b[1:]))
+
+
+def test_stream_lookup_refuses_a_cpu_tensor():
+    """A tensor that is on no GPU has no stream: the lookup by device index must
+    not fall through to the current device."""
+    import pytest
+    import torch
+
+    from nlearn_amd import _lib
+
+    with pytest.raises((ValueError, RuntimeError, AssertionError)):
+        _lib.stream_of(torch.zeros(4))
