@@ -558,11 +558,41 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
     if (kt + 1 < nfull) issue(nxt, kt + 1);
     compute(cur);
   };
+  // The smaller tiles take a whole K of up to 4096 (or a split's 2048) in one
+  // workgroup. They move their sums to a second set of registers every 512 k, so
+  // no chain of rounded additions is longer than the shortest split they stand
+  // in for (512 k): without it the fp32 result of K = 2048 was off by 2.7e-7
+  // against 1.85e-7 of the sum of two 1024-deep partials, with it by 1.31e-7.
+  constexpr bool kTwoLevel = BN == 64;
+  constexpr int kFlush = 512 / BKT;  // stages
+  f32x16 tot[kTwoLevel ? FM : 1][kTwoLevel ? FN : 1];
+  if constexpr (kTwoLevel) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) tot[i][j][r] = 0.f;
+  }
   if (nfull > 0) issue(st0, 0);
-  for (int kt = 0; kt < nfull; kt += 2) {
-    step(st0, st1, kt);
-    if (kt + 1 >= nfull) break;
-    step(st1, st0, kt + 1);
+  for (int kt0 = 0; kt0 < nfull; kt0 += kTwoLevel ? kFlush : nfull) {
+    const int kt1 = kTwoLevel ? min(nfull, kt0 + kFlush) : nfull;  // kFlush is even: the buffers keep their parity
+    for (int kt = kt0; kt < kt1; kt += 2) {
+      step(st0, st1, kt);
+      if (kt + 1 >= kt1) break;
+      step(st1, st0, kt + 1);
+    }
+    if constexpr (kTwoLevel) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            tot[i][j][r] += acc[i][j][r];
+            acc[i][j][r] = 0.f;
+          }
+    }
   }
   if (tail) {
     __syncthreads();
@@ -572,6 +602,14 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
     stage_masked<BN, BKT, B_KMAJ, NT>(g.B, g.ldb, n0, g.N, kt0, kend, sb + BM * BKT, tid);
     __syncthreads();
     compute(sb);
+  }
+  if constexpr (kTwoLevel) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] += tot[i][j][r];
   }
   const int frow = lane & 31;
   const int g4 = (lane >> 5) * 4;
@@ -1323,16 +1361,17 @@ Plan make_plan(int opA, int opB, int M, int N, int K, int epi) {
   // with 128-k stages (half the barriers and round trips, 64 KB of LDS) put four
   // times the workgroups on the chip and need no split up to K = 2048. Measured
   // (us, operands in the caches; 128 x 128 -> these):
-  //   NN 200 x 512 x 512     6.8 -> 3.9    NN 4096 x 512 x 512   7.3 -> 5.6
-  //   NN 2048 x 512 x 2048  20.3 -> 9.1    NN 4096 x 512 x 2048 24.3 -> 12.4
-  //   TN 512 x 2048 x 2048  19.5 -> 9.7    TN 512 x 512 x 4096  15.3 -> 10.2
+  //   NN 200 x 512 x 512     6.8 -> 4.2    NN 4096 x 512 x 512   7.3 -> 5.9
+  //   NN 2048 x 512 x 2048  20.3 -> 10.5   NN 4096 x 512 x 2048 24.3 -> 13.9
+  //   TN 512 x 2048 x 2048  19.5 -> 10.9   TN 512 x 512 x 4096  15.3 -> 11.1
+  // What is left is the CU's global -> LDS rate: 16 stages of 32 KB in 5.5 us.
   // The bound on their number is where two rounds of them lose: NN 2048 x 1536
-  // x 512 (768 tiles) 7.5 -> 8.1, 6000 x 512 x 2048 (752) 24.1 against 20.8 with
+  // x 512 (768 tiles) 7.5 -> 8.1, 6000 x 512 x 2048 (752) 24.1 against 21.3 with
   // 128 x 64 tiles. Those take over up to 256 tiles of 128 x 128 (2048 x 2048 x
-  // 512 10.3 -> 9.1, 8192 x 512 x 2048 23.4 -> 20.9, 1000 x 4096 x 1024 15.4 ->
-  // 13.1; beyond, 12000 x 512 x 2048 28.0 -> 31.8). Long reductions run on
+  // 512 10.3 -> 10.0, 8192 x 512 x 2048 23.4 -> 22.0, 1000 x 4096 x 1024 15.4 ->
+  // 12.3; beyond, 12000 x 512 x 2048 28.0 -> 31.8). Long reductions run on
   // 64 x 64 tiles, split, only over the smallest outputs (TN 512 x 512 x 16384
-  // 22.1 -> 19.9, NT 256 x 512 x 50256 38.7 -> 31.5; but 1024 x 512 x 50256
+  // 22.1 -> 20.3, NT 256 x 512 x 50256 38.7 -> 31.5; but 1024 x 512 x 50256
   // 89.6 -> 91.3).
   const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
   const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);

@@ -287,6 +287,24 @@ def test_gemm_small_product_tiles(dev, opA, opB, M, N, K):
     assert rel_l2(_np(ed), om._gelu_bwd(0.25 * ref, u.astype(np.float64), t)) <= 1e-5   # as the epilogue test's bound
 
 
+@pytest.mark.parametrize("M,N,K", [(512, 512, 2048), (512, 1536, 4096), (300, 1000, 1900), (2000, 1100, 4096)])
+def test_gemm_small_product_tiles_sum_in_short_chains(dev, M, N, K):
+    """A whole K in one workgroup must not add up less exactly than the split it
+    replaced. A chain of n rounded additions of random signs errs by a share of
+    2^-24 sqrt(n) of its result: measured 1.3e-7 for chains of 512, as the
+    128 x 128 tiles give at K = 512, and sqrt(4) times that, 2.7e-7, for one chain
+    of 2048. The bound is the chain of 1024 that the former split had, 1.9e-7."""
+    import torch
+    from nlearn_amd.kernels.gemm import gemm_raw
+
+    gen = torch.Generator(device=dev).manual_seed(K)
+    A = torch.randn((K, M), generator=gen, device=dev).to(torch.bfloat16)
+    B = torch.randn((K, (N + 7) // 8 * 8), generator=gen, device=dev).to(torch.bfloat16)[:, :N]
+    ref = A.double().t().contiguous() @ B.double()
+    err = float((gemm_raw(A, B, "T", "N").double() - ref).norm() / ref.norm())
+    assert err <= 1.9e-7
+
+
 @pytest.mark.parametrize("opB,M,N,K,out", [("N", 4100, 4000, 128, "f32"), ("N", 4100, 4000, 256, "bf16"),
                                            ("T", 4097, 4033, 384, "f32"), ("T", 16384, 2048, 512, "bf16"),
                                            ("N", 16384, 1536, 512, "bf16")])
