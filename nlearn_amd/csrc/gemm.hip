@@ -558,12 +558,17 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
     if (kt + 1 < nfull) issue(nxt, kt + 1);
     compute(cur);
   };
-  // The smaller tiles take a whole K of up to 4096 (or a split's 2048) in one
-  // workgroup. They move their sums to a second set of registers every 512 k, so
-  // no chain of rounded additions is longer than the shortest split they stand
-  // in for (512 k): without it the fp32 result of K = 2048 was off by 2.7e-7
-  // against 1.85e-7 of the sum of two 1024-deep partials, with it by 1.31e-7.
+  // The smaller tiles take a whole K, or a long split's share of it, in one
+  // workgroup. Where the sums leave in fp32 (an fp32 C, a split's partials) they
+  // move to a second set of registers every 512 k, so no chain of rounded
+  // additions is longer than the shortest split they stand in for (512 k):
+  // without it the fp32 result of K = 2048 was off by 2.7e-7 against 1.85e-7 of
+  // the sum of two 1024-deep partials, with it by 1.31e-7. A bf16 C of one
+  // workgroup per tile keeps the single chain of the larger tiles (the rounding
+  // to bf16 is 10^4 times those errors): its bits then do not depend on which
+  // tile a row count selects, as the chunked LM head promises.
   constexpr bool kTwoLevel = BN == 64;
+  const bool two_level = kTwoLevel && (sizeof(OutT) == 4 || g.ws);
   constexpr int kFlush = 512 / BKT;  // stages
   f32x16 tot[kTwoLevel ? FM : 1][kTwoLevel ? FN : 1];
   if constexpr (kTwoLevel) {
@@ -575,23 +580,25 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
         for (int r = 0; r < 16; ++r) tot[i][j][r] = 0.f;
   }
   if (nfull > 0) issue(st0, 0);
-  for (int kt0 = 0; kt0 < nfull; kt0 += kTwoLevel ? kFlush : nfull) {
-    const int kt1 = kTwoLevel ? min(nfull, kt0 + kFlush) : nfull;  // kFlush is even: the buffers keep their parity
+  for (int kt0 = 0; kt0 < nfull; kt0 += two_level ? kFlush : nfull) {
+    const int kt1 = two_level ? min(nfull, kt0 + kFlush) : nfull;  // kFlush is even: the buffers keep their parity
     for (int kt = kt0; kt < kt1; kt += 2) {
       step(st0, st1, kt);
       if (kt + 1 >= kt1) break;
       step(st1, st0, kt + 1);
     }
     if constexpr (kTwoLevel) {
+      if (two_level) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
+          for (int j = 0; j < FN; ++j)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            tot[i][j][r] += acc[i][j][r];
-            acc[i][j][r] = 0.f;
-          }
+            for (int r = 0; r < 16; ++r) {
+              tot[i][j][r] += acc[i][j][r];
+              acc[i][j][r] = 0.f;
+            }
+      }
     }
   }
   if (tail) {
@@ -604,12 +611,14 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
     compute(sb);
   }
   if constexpr (kTwoLevel) {
+    if (two_level) {
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+      for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
+        for (int j = 0; j < FN; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] += tot[i][j][r];
+          for (int r = 0; r < 16; ++r) acc[i][j][r] += tot[i][j][r];
+    }
   }
   const int frow = lane & 31;
   const int g4 = (lane >> 5) * 4;
