@@ -189,6 +189,8 @@ int nl_flash_attention_bwd_dkdv(void* stream, int batch, int heads, int seq, int
 
 /* Whole backward (D, dK/dV and dQ) in one call. `ws` is a caller-owned
  * device workspace of nl_flash_attention_bwd_ws_bytes() bytes (holds D).
+ * dQ may be written over Q, O or dO, dK or dV over O (the same address and
+ * strides); no output may overlap an input in any other way.
  * Replaces _flash_bwd_rule (attention.py:111-128). */
 size_t nl_flash_attention_bwd_ws_bytes(int batch, int heads, int seq);
 int nl_flash_attention_bwd(void* stream, int batch, int heads, int seq, int d_head,

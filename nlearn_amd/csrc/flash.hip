@@ -33,8 +33,10 @@
 //     partial results are combined in LDS. What bounds such a call is the chain
 //     of blocks of its longest tile on a chip that is not full.
 #include <type_traits>
+#include <algorithm>
 #include <atomic>
 #include <mutex>
+#include <utility>
 
 #include "common.h"
 
@@ -858,6 +860,19 @@ int check_op(const void* p, const nl_attn_stride& s, const char* name) {
     return nl_set_error(NL_EALIGN, std::string("flash: ") + name + " strides must be multiples of 8 (row >= 64)");
   return NL_OK;
 }
+// whether the address ranges of two [B][H][S][64] operands meet
+bool ranges_meet(int B, int H, int S, const void* p, const nl_attn_stride& sp, const void* q, const nl_attn_stride& sq) {
+  auto range = [&](const void* base, const nl_attn_stride& s) {
+    int64_t lo = 0, hi = 64;
+    for (const int64_t last : {(B - 1) * s.batch, (H - 1) * s.head, (S - 1) * s.row}) {
+      lo += std::min<int64_t>(last, 0);
+      hi += std::max<int64_t>(last, 0);
+    }
+    return std::pair<intptr_t, intptr_t>((intptr_t)base + lo * 2, (intptr_t)base + hi * 2);
+  };
+  const auto a = range(p, sp), b = range(q, sq);
+  return a.first < b.second && b.first < a.second;
+}
 
 }  // namespace
 }  // namespace nl
@@ -1027,8 +1042,10 @@ extern "C" int nl_flash_attention_bwd(void* stream, int batch, int heads, int se
   // reads: the preprocess launch (4 us) is a tenth of such a backward. On a full
   // chip D's O rows would only lengthen the start of every dQ workgroup: at 32 x
   // 512 x 8 heads forward + backward took 100.0 us against 97.6 with the
-  // preprocess (at 4 x 4096, 349 against 350).
-  if (ks == 1) {
+  // preprocess (at 4 x 4096, 349 against 350). A dQ that is written over Q or dO
+  // has to come last, since dK/dV reads all of both; a dQ workgroup reads only its
+  // own rows of them, before it writes these.
+  if (ks == 1 || ranges_meet(batch, heads, seq, dQ, sdq, Q, sq) || ranges_meet(batch, heads, seq, dQ, sdq, dO, sdo)) {
     NL_TRY(nl_flash_attention_bwd_preprocess(stream, batch, heads, seq, d_head, O, so, dO, sdo, D));
     NL_TRY(nl_flash_attention_bwd_dkdv(stream, batch, heads, seq, d_head, scale, causal, Q, sq, K, sk, V, sv, dO, sdo,
                                        L, D, dK, sdk, dV, sdv));
@@ -1095,8 +1112,8 @@ extern "C" int nl_flash_attention_bwd_noalloc(void* stream, int batch, int heads
                                        std::to_string(NL_FLASH_BWD_NOALLOC_MAX_ROWS) + ")");
   float* D = nullptr;
   NL_TRY(scratch_on_current_device(&D));
-  // D is written whole by the preprocess before dK/dV and dQ read it, so the
-  // array needs no clearing between calls.
+  // D is written whole (by the preprocess, or by dQ when it comes first) before
+  // dK/dV reads it, so the array needs no clearing between calls.
   return nl_flash_attention_bwd(stream, batch, heads, seq, d_head, scale, causal, Q, sq, K, sk, V, sv, O, so, dO, sdo,
                                 L, dQ, sdq, dK, sdk, dV, sdv, D);
 }

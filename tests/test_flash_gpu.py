@@ -113,6 +113,25 @@ def test_flash_tile_counts_on_both_sides(dev, B, H, S, causal):
     _check_against_oracle((O, L, dq, dk, dv), f32, B, H, S, causal)
 
 
+@pytest.mark.parametrize("B,H,S", [(2, 3, 97), (1, 2, 300), (52, 5, 97)])
+@pytest.mark.parametrize("out,over", [("dq", "q"), ("dq", "O"), ("dq", "do"), ("dk", "O"), ("dv", "O")])
+def test_flash_bwd_over_an_input(dev, B, H, S, out, over):
+    """dQ written over Q, O or dO, and dK or dV over O, leave all three gradients
+    as with buffers of their own, bit for bit (few tiles, and more than 256)."""
+    import torch
+    from nlearn_amd.attention import flash_bwd_raw4, flash_fwd_raw4
+
+    (q, k, v, do), _ = _rand_case(dev, B, H, S, seed=S)
+    O, L = flash_fwd_raw4(q, k, v, causal=True)
+    ref = flash_bwd_raw4(q, k, v, O, do, L)
+    t = {"q": q.clone(), "O": O.clone(), "do": do.clone()}
+    got = flash_bwd_raw4(t["q"], k, v, t["O"], t["do"], L, **{out: t[over]})
+    torch.cuda.synchronize()
+    assert got[("dq", "dk", "dv").index(out)].data_ptr() == t[over].data_ptr()
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("B,H,S", [(1, 2, 545), (2, 1, 1024)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_flash_scores_growing_along_the_keys(dev, B, H, S, causal):
