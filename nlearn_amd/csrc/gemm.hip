@@ -559,16 +559,15 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
     compute(cur);
   };
   // The smaller tiles take a whole K, or a long split's share of it, in one
-  // workgroup. Where the sums leave in fp32 (an fp32 C, a split's partials) they
-  // move to a second set of registers every 512 k, so no chain of rounded
-  // additions is longer than the shortest split they stand in for (512 k):
-  // without it the fp32 result of K = 2048 was off by 2.7e-7 against 1.85e-7 of
-  // the sum of two 1024-deep partials, with it by 1.31e-7. A bf16 C of one
-  // workgroup per tile keeps the single chain of the larger tiles (the rounding
-  // to bf16 is 10^4 times those errors): its bits then do not depend on which
-  // tile a row count selects, as the chunked LM head promises.
+  // workgroup. They move their sums to a second set of registers every 512 k, so
+  // no chain of rounded additions is longer than the shortest split they stand
+  // in for (512 k): without it the fp32 result of K = 2048 was off by 2.7e-7
+  // against 1.85e-7 of the sum of two 1024-deep partials, with it by 1.31e-7.
+  // A bf16 C of K <= 1024 keeps the single chain of the larger tiles (the
+  // rounding to bf16 is 10^4 times those errors): its bits then do not depend on
+  // which tile a row count selects, as the chunked LM head promises.
   constexpr bool kTwoLevel = BN == 64;
-  const bool two_level = kTwoLevel && (sizeof(OutT) == 4 || g.ws);
+  const bool two_level = kTwoLevel && (sizeof(OutT) == 4 || g.ws || g.K > 1024);
   constexpr int kFlush = 512 / BKT;  // stages
   f32x16 tot[kTwoLevel ? FM : 1][kTwoLevel ? FN : 1];
   if constexpr (kTwoLevel) {

@@ -174,11 +174,11 @@ class _LMHeadCE(torch.autograd.Function):
     over the logits), in row chunks. With more than one chunk, each chunk's CE
     runs on a second stream while the GEMM computes the next chunk, so the
     HBM-bound CE overlaps the MFMA-bound GEMM. Rows are independent in both
-    kernels, and the CE scale is 1/M of all rows. Up to d = 2048 the logits GEMM
+    kernels, and the CE scale is 1/M of all rows. Up to d = 1024 the logits GEMM
     adds every element up in one chain over k, whatever tile its row count
     selects, so every value equals the unchunked linear + cross_entropy bit for
-    bit (a deeper product over few tiles is split over k by its own row count:
-    there the chunks may differ from the whole in the last fp32 bit before the
+    bit (a deeper sum is divided over k as its tile has it: there a chunk's
+    logits may differ from the whole's where the last fp32 bits decide the
     rounding to bf16). The backward is linear's, from dlogits scaled by the
     cotangent."""
 
@@ -234,7 +234,7 @@ def lm_head_cross_entropy(X: torch.Tensor, W: torch.Tensor, targets: torch.Tenso
                           overlap: bool = True) -> torch.Tensor:
     """Mean CE of logits = X . W (X [..., d] bf16, W [d, V]) against ``targets``,
     equal to ``cross_entropy(linear(X, W), targets, inplace=True)`` bit for
-    bit up to d = 2048; with ``chunks`` > 1 row chunks, the CE of one chunk
+    bit up to d = 1024; with ``chunks`` > 1 row chunks, the CE of one chunk
     overlaps the GEMM of the next (see _LMHeadCE) unless ``overlap`` is False
     (every kernel then runs on the current stream, in the same order)."""
     if X.dim() < 2 or W.dim() != 2:
