@@ -389,7 +389,7 @@ __device__ __forceinline__ void ce_combine(float& m, float& s, float m2, float s
   m = mn;
 }
 
-template <int BM, int BN, int BKT, bool A_KMAJ, bool B_KMAJ, typename OutT, int EPI>
+template <int BM, int BN, int BKT, bool A_KMAJ, bool B_KMAJ, typename OutT, int EPI, bool kTwoLevel = BN == 64>
 __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
                              (BM * BN >= 65536) ? 1 : 2) void gemm2_kernel(GemmArgs g) {
   // 256 x 256 tiles run 8 waves (2 x 4), the others 4 (2 x 2); every wave
@@ -563,11 +563,7 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
   // no chain of rounded additions is longer than the shortest split they stand
   // in for (512 k): without it the fp32 result of K = 2048 was off by 2.7e-7
   // against 1.85e-7 of the sum of two 1024-deep partials, with it by 1.31e-7.
-  // A bf16 C of K <= 1024 keeps the single chain of the larger tiles (the
-  // rounding to bf16 is 10^4 times those errors): its bits then do not depend on
-  // which tile a row count selects, as the chunked LM head promises.
-  constexpr bool kTwoLevel = BN == 64;
-  const bool two_level = kTwoLevel && (sizeof(OutT) == 4 || g.ws || g.K > 1024);
+  // (launch_cfg says where they keep one chain.)
   constexpr int kFlush = 512 / BKT;  // stages
   f32x16 tot[kTwoLevel ? FM : 1][kTwoLevel ? FN : 1];
   if constexpr (kTwoLevel) {
@@ -579,25 +575,23 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
         for (int r = 0; r < 16; ++r) tot[i][j][r] = 0.f;
   }
   if (nfull > 0) issue(st0, 0);
-  for (int kt0 = 0; kt0 < nfull; kt0 += two_level ? kFlush : nfull) {
-    const int kt1 = two_level ? min(nfull, kt0 + kFlush) : nfull;  // kFlush is even: the buffers keep their parity
+  for (int kt0 = 0; kt0 < nfull; kt0 += kTwoLevel ? kFlush : nfull) {
+    const int kt1 = kTwoLevel ? min(nfull, kt0 + kFlush) : nfull;  // kFlush is even: the buffers keep their parity
     for (int kt = kt0; kt < kt1; kt += 2) {
       step(st0, st1, kt);
       if (kt + 1 >= kt1) break;
       step(st1, st0, kt + 1);
     }
     if constexpr (kTwoLevel) {
-      if (two_level) {
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+      for (int i = 0; i < FM; ++i)
 #pragma unroll
-          for (int j = 0; j < FN; ++j)
+        for (int j = 0; j < FN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              tot[i][j][r] += acc[i][j][r];
-              acc[i][j][r] = 0.f;
-            }
-      }
+          for (int r = 0; r < 16; ++r) {
+            tot[i][j][r] += acc[i][j][r];
+            acc[i][j][r] = 0.f;
+          }
     }
   }
   if (tail) {
@@ -610,14 +604,12 @@ __global__ __launch_bounds__((BM * BN >= 65536) ? 512 : 256,
     compute(sb);
   }
   if constexpr (kTwoLevel) {
-    if (two_level) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
+      for (int j = 0; j < FN; ++j)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][j][r] += tot[i][j][r];
-    }
+        for (int r = 0; r < 16; ++r) acc[i][j][r] += tot[i][j][r];
   }
   const int frow = lane & 31;
   const int g4 = (lane >> 5) * 4;
@@ -1199,6 +1191,8 @@ __global__ __launch_bounds__(NWV * 64, NWV == 8 ? 1 : 2) void gemm_persist_kerne
 #define NL_SALL(BM, BN, BKT) NL_S3(BM, BN, BKT, NL_EPI_NONE) NL_S3(BM, BN, BKT, NL_EPI_BIAS) NL_S3(BM, BN, BKT, NL_EPI_BIAS_GELU) NL_S3(BM, BN, BKT, NL_EPI_DGELU)
 NL_SALL(64, 64, 128)
 NL_SALL(128, 64, 64)
+template __global__ void gemm2_kernel<64, 64, 128, true, false, uint16_t, NL_EPI_NONE, false>(GemmArgs);
+template __global__ void gemm2_kernel<128, 64, 64, true, false, uint16_t, NL_EPI_NONE, false>(GemmArgs);
 NL_I8(NL_EPI_NONE)
 NL_I8(NL_EPI_BIAS)
 NL_I8(NL_EPI_BIAS_GELU)
@@ -1443,6 +1437,21 @@ void launch_cfg(GemmArgs g, const Plan& p, hipStream_t st) {
     }
     if constexpr (AK || !BK_) {
       if (p.tile == kTile64 || p.tile == kTile128x64) {
+        // A bf16 NN product of K <= 1024 without an epilogue (logits among them) has
+        // the one chain over K of the larger tiles, so that its bits do not depend
+        // on the tile a row count selects, as the chunked LM head promises. The
+        // rounding to bf16 is 10^4 times what the chain's length adds.
+        if constexpr (AK && !BK_ && sizeof(OutT) == 2) {
+          if (g.epi == NL_EPI_NONE && !g.ws && g.K <= 1024) {
+            if (p.tile == kTile64)
+              hipLaunchKernelGGL((gemm2_kernel<64, 64, 128, AK, BK_, OutT, NL_EPI_NONE, false>), dim3(grid), dim3(256),
+                                 0, st, g);
+            else
+              hipLaunchKernelGGL((gemm2_kernel<128, 64, 64, AK, BK_, OutT, NL_EPI_NONE, false>), dim3(grid), dim3(256),
+                                 0, st, g);
+            return;
+          }
+        }
         auto go = [&](auto e) {
           constexpr int E = decltype(e)::value;
           if (p.tile == kTile64)
