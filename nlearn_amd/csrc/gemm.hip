@@ -1289,7 +1289,9 @@ int cu_count() {
 
 enum Tile { kTile64, kTile128x64, kTile128, kTile256x128, kTile256 };
 
-// Tile configuration and K split of one product (shared by the workspace query).
+// Tile configuration and K split of one product (shared by the workspace query:
+// the split depends on neither the epilogue nor the output type where it is below
+// the 256 x 256 tiles' line).
 struct Plan {
   Tile tile;
   int tiles;
@@ -1299,13 +1301,15 @@ struct Plan {
   size_t ws_bytes;
 };
 
-Plan make_plan(int opA, int opB, int M, int N, int K, int epi) {
+// The products that small_plan leaves.
+Plan large_plan(int opA, int opB, int M, int N, int K, int epi) {
   Plan p;
   p.tile = kTile128;
   p.tiles = (int)((int64_t)((M + 127) / 128) * ((N + 127) / 128));
   p.splits = 1;
   p.k_chunk = K > 0 ? K : 1;
-  // skinny outputs with a long reduction (weight gradients, K = tokens): split K.
+  // skinny outputs with a long reduction (weight gradients, K = tokens; above 4096
+  // in all forms but TT): split K.
   // X^T dY (TN) products: a power-of-two split towards 512 workgroups, >= 1024 k
   // per split (measured on MI355X at the model's weight-gradient shapes: 10-20%
   // faster than the generic rule below); others: ~640 workgroups, >= 512 k.
@@ -1357,46 +1361,83 @@ Plan make_plan(int opA, int opB, int M, int N, int K, int epi) {
       p.splits = (K + chunk - 1) / chunk;
     }
   }
-  // Products too small to give every CU two 128 x 128 tiles (a few hundred to a
-  // few thousand tokens): they wait on their k stages, one DMA round trip after
-  // the other, and on the split's second launch, not on MFMAs. 64 x 64 tiles
-  // with 128-k stages (half the barriers and round trips, 64 KB of LDS) put four
-  // times the workgroups on the chip and need no split up to K = 2048. Measured
-  // (us, operands in the caches; 128 x 128 -> these):
-  //   NN 200 x 512 x 512     6.8 -> 4.2    NN 4096 x 512 x 512   7.3 -> 5.9
-  //   NN 2048 x 512 x 2048  20.3 -> 10.5   NN 4096 x 512 x 2048 24.3 -> 13.9
-  //   TN 512 x 2048 x 2048  19.5 -> 10.9   TN 512 x 512 x 4096  15.3 -> 11.1
-  // What is left is the CU's global -> LDS rate: 16 stages of 32 KB in 5.5 us.
-  // The bound on their number is where two rounds of them lose: NN 2048 x 1536
-  // x 512 (768 tiles) 7.5 -> 8.1, 6000 x 512 x 2048 (752) 24.1 against 21.3 with
-  // 128 x 64 tiles. Those take over up to 256 tiles of 128 x 128 (2048 x 2048 x
-  // 512 10.3 -> 10.0, 8192 x 512 x 2048 23.4 -> 22.0, 1000 x 4096 x 1024 15.4 ->
-  // 12.3; beyond, 12000 x 512 x 2048 28.0 -> 31.8). Long reductions run on
-  // 64 x 64 tiles, split, only over the smallest outputs (TN 512 x 512 x 16384
-  // 22.1 -> 20.3, NT 256 x 512 x 50256 38.7 -> 31.5; but 1024 x 512 x 50256
-  // 89.6 -> 91.3).
+  return p;
+}
+
+// Products too small to give every CU two 128 x 128 tiles (a few hundred to a
+// few thousand tokens): they wait on their k stages, one DMA round trip after
+// the other, and on the split's second launch, not on MFMAs. 64 x 64 tiles with
+// 128-k stages (half the barriers and round trips, 64 KB of LDS) put four times
+// the workgroups on the chip and need no split up to K = 2048. Measured (us,
+// operands in the caches; 128 x 128 -> these):
+//   NN 200 x 512 x 512     6.8 -> 4.2    NN 4096 x 512 x 512   7.3 -> 5.9
+//   NN 2048 x 512 x 2048  20.3 -> 10.5   NN 4096 x 512 x 2048 24.3 -> 13.9
+//   TN 512 x 2048 x 2048  19.5 -> 10.9   TN 512 x 512 x 4096  15.3 -> 11.1
+// What is left is the CU's global -> LDS rate: 16 stages of 32 KB in 5.5 us.
+// Where the lines lie:
+// * Two rounds of 64 x 64 tiles lose (6000 x 512 x 2048, 752 tiles: 24.1 against
+//   21.3 with 128 x 64).
+// * A k-contiguous operand whose K leaves 64 after whole 128-k stages pays for
+//   the register-staged tail what two 64-k stages do not: NN 4096 x 512 at K =
+//   64, 192, 320, 576: 4.3, 5.1, 6.0, 7.8 with 128 x 128 against 4.8, 5.8, 6.3,
+//   7.4; 2048 x 512 at 192 and 320: 5.0, 5.9 against 5.4, 5.7. (A GELU epilogue
+//   over four times the workgroups gains more: 6.7 against 5.8 at K = 64. An fp32
+//   C lies between: 4096 x 512 at 192 and 320: 6.0, 6.9 against 6.2, 6.6.)
+// * Long reductions take them, split, over the smallest outputs, as long as their
+//   operand traffic (twice that of 128 x 128 tiles) is not what counts: TN 512 x
+//   512 at K = 16384, 32768, 50256, 131072: 22.7, 33.1, 40.6, 88 with the larger
+//   tiles against 20.5, 32.3, 45.0, 117 with these, TN 192 x 512 at 131072 and
+//   262144: 51, 104 against 45, 115; NT 512 x 512 at 50256, 65536, 100000: 56, 57,
+//   89 against 52, 54, 89, NT 192 x 512 at 262144 129 against 112. Splits of 2048,
+//   or shorter ones (>= 1024) while those leave CUs without a workgroup: NN 64 x
+//   64 x 8192 10.3 in 8 splits, 12.6 in 4 (11.4 as 128 x 128 in 16 of 512).
+// * 128 x 64 tiles up to 256 tiles of 128 x 128 where those would split K (3000 x
+//   1024 x 1024 23.9 -> 12.4, TN 768 x 3072 x 2048 27.7 -> 20.6), in the TN form at
+//   every K (1024 x 4096 x 333 9.8 -> 9.1), and where twice the workgroups overlap
+//   an fp32 or GELU epilogue (2048 x 2048 x 512: GELU 11.6 -> 11.0, GELU' 10.9 ->
+//   10.2, fp32 10.1 -> 9.4) or a long loop (8192 x 512 x 2048 25.2 -> 23.7, 16384 x
+//   256 x 1024 14.8 -> 13.3). A short bf16 product alone is the other way round
+//   (NN 8192 x 512 x 512 7.9 -> 8.5, 1024 x 4096 x 1024 12.9 -> 13.5) unless much of
+//   the chip is idle (NT 3000 x 768 x 768, 144 tiles: 9.7 -> 9.3), and so is a K
+//   tail of a k-contiguous operand (1000 x 4096 x 1000 14.7 -> 16.7).
+bool small_plan(int opA, int opB, int M, int N, int K, int epi, bool f32, Plan& p) {
+  if ((opA == NL_OP_T && opB == NL_OP_T) || K <= 0) return false;
+  const bool tn = opA == NL_OP_T;
+  const bool gelu = epi == NL_EPI_BIAS_GELU || epi == NL_EPI_DGELU;
   const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
   const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-  if (!(opA == NL_OP_T && opB == NL_OP_T) && K > 0) {
-    if (t64 <= (K <= 4096 ? 512 : 64)) {
-      p.tile = kTile64;
-      p.tiles = (int)t64;
-      p.splits = 1;
-      p.k_chunk = K;
-      const int per = K <= 4096 ? 1024 : 2048;
-      const int sp = std::min(512 / p.tiles, (K + per - 1) / per);
-      if (K > 2048 && sp > 1) {
-        const int chunk = ((K + sp - 1) / sp + 127) / 128 * 128;
-        p.k_chunk = chunk;
-        p.splits = (K + chunk - 1) / chunk;
-      }
-    } else if (t128 <= 256 && K <= 4096) {
-      p.tile = kTile128x64;
-      p.tiles = (int)((int64_t)((M + 127) / 128) * ((N + 63) / 64));
-      p.splits = 1;
-      p.k_chunk = K;
+  p.splits = 1;
+  p.k_chunk = K;
+  // products of tiles and K (operand traffic) up to which a long reduction comes here
+  const int64_t reach = (int64_t)(tn ? (t64 <= 24 ? 3 : 2) : (t64 <= 24 ? 8 : 4)) << 20;
+  if (K <= 4096 ? t64 <= 512 : t64 <= 64 && t64 * K <= reach) {
+    const int tail_k = f32 ? (t64 > 256 ? 192 : 0) : t64 > 256 ? 448 : 192;
+    if (!tn && !gelu && K % 128 == 64 && K <= tail_k) return false;
+    p.tile = kTile64;
+    p.tiles = (int)t64;
+    auto parts = [&](int per) { return (K + per - 1) / per; };
+    const int sp = K <= 4096 ? std::min(512 / p.tiles, parts(1024))
+                             : std::min(512 / p.tiles, std::max(parts(2048), std::min(256 / p.tiles, parts(1024))));
+    if (K > 2048 && sp > 1) {
+      const int chunk = ((K + sp - 1) / sp + 127) / 128 * 128;
+      p.k_chunk = chunk;
+      p.splits = (K + chunk - 1) / chunk;
     }
+    return true;
   }
+  const bool would_split = K >= 1024 && t128 < 256;
+  const bool long_k = K > 1024 || (K == 1024 && N <= 256) || (K >= 768 && opB == NL_OP_T) || (K >= 512 && t128 <= 160);
+  const bool epilogue = epi == NL_EPI_DGELU || (K >= 128 && (f32 || epi != NL_EPI_NONE));
+  const bool worth = K % 64 == 0 && (long_k || epilogue);
+  if (t128 > 256 || K > 4096 || !(tn || would_split || worth)) return false;
+  p.tile = kTile128x64;
+  p.tiles = (int)((int64_t)((M + 127) / 128) * ((N + 63) / 64));
+  return true;
+}
+
+Plan make_plan(int opA, int opB, int M, int N, int K, int epi, bool f32) {
+  Plan p;
+  if (!small_plan(opA, opB, M, N, K, epi, f32, p)) p = large_plan(opA, opB, M, N, K, epi);
   p.ldw = ((int64_t)N + 7) / 8 * 8;
   p.ws_bytes = p.splits > 1 ? (size_t)p.splits * M * p.ldw * sizeof(float) : 0;
   return p;
@@ -1765,9 +1806,9 @@ extern "C" size_t nl_gemm_ws_bytes(int opA, int opB, int M, int N, int K) {
   g.ldb = ((opB == NL_OP_N ? (int64_t)N : K) + 7) / 8 * 8;
   g.ldc = ((int64_t)N + 7) / 8 * 8;
   g.epi = NL_EPI_NONE;
-  size_t most = make_plan(opA, opB, M, N, K, NL_EPI_NONE).ws_bytes;
+  size_t most = make_plan(opA, opB, M, N, K, NL_EPI_NONE, true).ws_bytes;
   for_each_subproduct(opA, opB, g, NL_DTYPE_F32, [&](const GemmArgs& s) {
-    most = std::max(most, make_plan(opA, opB, s.M, s.N, s.K, NL_EPI_NONE).ws_bytes);
+    most = std::max(most, make_plan(opA, opB, s.M, s.N, s.K, NL_EPI_NONE, true).ws_bytes);
     return NL_OK;
   });
   return most;
@@ -1823,7 +1864,7 @@ extern "C" int nl_gemm_fused(void* stream, int opA, int opB, int M, int N, int K
   int rc = for_each_subproduct(opA, opB, g, c_dtype, [](const GemmArgs&) { return NL_OK; });
   if (rc) return rc;
   rc = for_each_subproduct(opA, opB, g, c_dtype, [&](const GemmArgs& s) {
-    Plan p = make_plan(opA, opB, s.M, s.N, s.K, s.epi);
+    Plan p = make_plan(opA, opB, s.M, s.N, s.K, s.epi, c_dtype == NL_DTYPE_F32);
     if (p.splits > 1 && (!ws || ws_bytes < p.ws_bytes || ((uintptr_t)ws & 15) != 0)) {
       // no (usable) workspace: one workgroup per tile over the whole K range
       p.splits = 1;
