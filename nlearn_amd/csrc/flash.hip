@@ -834,23 +834,38 @@ int check_common(int B, int H, int S, int d, int causal) {
   if (H > 65535 || B > 65535) return nl_set_error(NL_EINVAL, "flash: batch and heads must be <= 65535");
   return NL_OK;
 }
-// Wave groups per workgroup (KS) and the grid of 128 / KS-row tiles. Two groups
-// (64-row tiles, each group every other block of the streamed side) pay while
-// all their workgroups are resident at once: their LDS allows two per CU, so up
-// to 256 tiles of 128 rows. Measured, one group -> two (us; forward, backward):
-//   16 tiles (1 x 200 x 8 heads)   6.1 -> 5.2    18.5 -> 14.3
-//   112 (2 x 777 x 8)             12.8 -> 9.7    39.3 -> 25.5
-//   256 (8 x 512 x 8)             10.3 -> 8.6    30.3 -> 23.4
-//   256 (1 x 4096 x 8)            50.2 -> 36.4  155.2 -> 94.6
+// Wave groups per workgroup (KS): two groups (64-row tiles, each group every other
+// block of the streamed side) pay while all their workgroups are resident at once:
+// their LDS allows two per CU, so up to 256 tiles of 128 rows. Measured, one group
+// -> two (us; forward, backward):
+//   16 tiles (1 x 200 x 8 heads)   6.5 -> 5.6    19.9 -> 14.6
+//   112 (2 x 777 x 8)             13.0 -> 9.9    40.6 -> 26.2
+//   256 (8 x 512 x 8)             10.2 -> 8.6    32.6 -> 24.0
+//   256 (1 x 4096 x 8)            50.7 -> 35.9  157.2 -> 99.3
 //   512 (16 x 512 x 8)            13.0 -> 14.2   37.5 -> 43.7
 // Four groups of 32 rows (128 KB of LDS, one workgroup per CU) gained on two
 // only under 64 tiles, at most 10%: not kept.
+// The forward does less per block than the merge and the second set of buffers
+// cost where a group has a block or two: one group up to 64 rows (1 x 64 x 8 4.1
+// against 4.6 with two) and, once two workgroups share a CU, below 256 rows
+// causal and 768 not (32 x 128 x 8 5.8 against 6.3, 8 x 512 x 8 not causal 9.9
+// against 10.4; from there 16 x 256 x 8 causal 7.2 -> 6.8, 4 x 768 x 8 not causal
+// 12.7 -> 12.5). The backward is never slower with two (1 x 64 x 8 12.0, 12.0).
 constexpr int64_t kTwoGroupTiles = 256;
-int tile_grid(int batch, int heads, int seq, dim3& grid, int& ks) {
-  auto wgs = [&](int k) { return (int64_t)((seq + kRows / k - 1) / (kRows / k)) * heads * batch; };
-  ks = wgs(1) <= kTwoGroupTiles ? 2 : 1;
-  if (wgs(ks) >= ((int64_t)1 << 31)) return nl_set_error(NL_EUNSUPPORTED, "flash: too many tiles");
-  grid = dim3((unsigned)wgs(ks));
+constexpr int64_t kCus = 256;
+int64_t tiles_of(int batch, int heads, int seq, int ks) {
+  return (int64_t)((seq + kRows / ks - 1) / (kRows / ks)) * heads * batch;
+}
+int bwd_groups(int batch, int heads, int seq) { return tiles_of(batch, heads, seq, 1) <= kTwoGroupTiles ? 2 : 1; }
+int fwd_groups(int batch, int heads, int seq, int causal) {
+  if (seq <= kRows / 2 || tiles_of(batch, heads, seq, 1) > kTwoGroupTiles) return 1;
+  return tiles_of(batch, heads, seq, 2) <= kCus || seq >= (causal ? 256 : 768) ? 2 : 1;
+}
+// the grid of 128 / ks-row tiles
+int tile_grid(int batch, int heads, int seq, int ks, dim3& grid) {
+  const int64_t wgs = tiles_of(batch, heads, seq, ks);
+  if (wgs >= ((int64_t)1 << 31)) return nl_set_error(NL_EUNSUPPORTED, "flash: too many tiles");
+  grid = dim3((unsigned)wgs);
   return NL_OK;
 }
 int check_op(const void* p, const nl_attn_stride& s, const char* name) {
@@ -910,8 +925,8 @@ extern "C" int nl_flash_attention_fwd(void* stream, int batch, int heads, int se
   a.H = heads;
   a.B = batch;
   dim3 grid;
-  int ks;
-  NL_TRY(tile_grid(batch, heads, seq, grid, ks));
+  const int ks = fwd_groups(batch, heads, seq, causal);
+  NL_TRY(tile_grid(batch, heads, seq, ks, grid));
   const hipStream_t st = (hipStream_t)stream;
   if (ks == 2) hipLaunchKernelGGL(flash_fwd_kernel<2>, grid, dim3(kThreads), 0, st, a);
   else hipLaunchKernelGGL(flash_fwd_kernel<1>, grid, dim3(kThreads), 0, st, a);
@@ -965,8 +980,8 @@ static int launch_dq(void* stream, int batch, int heads, int seq, BwdArgs& a) {
   a.H = heads;
   a.B = batch;
   dim3 grid;
-  int ks;
-  NL_TRY(tile_grid(batch, heads, seq, grid, ks));
+  const int ks = bwd_groups(batch, heads, seq);
+  NL_TRY(tile_grid(batch, heads, seq, ks, grid));
   const hipStream_t st = (hipStream_t)stream;
   if (ks == 1) hipLaunchKernelGGL((flash_bwd_dq_kernel<1, false>), grid, dim3(kThreads), 0, st, a);
   else if (a.Dout) hipLaunchKernelGGL((flash_bwd_dq_kernel<2, true>), grid, dim3(kThreads), 0, st, a);
@@ -1004,8 +1019,8 @@ extern "C" int nl_flash_attention_bwd_dkdv(void* stream, int batch, int heads, i
   a.H = heads;
   a.B = batch;
   dim3 grid;
-  int ks;
-  NL_TRY(tile_grid(batch, heads, seq, grid, ks));
+  const int ks = bwd_groups(batch, heads, seq);
+  NL_TRY(tile_grid(batch, heads, seq, ks, grid));
   const hipStream_t st = (hipStream_t)stream;
   if (ks == 2) hipLaunchKernelGGL(flash_bwd_dkdv_kernel<2>, grid, dim3(kThreads), 0, st, a);
   else hipLaunchKernelGGL(flash_bwd_dkdv_kernel<1>, grid, dim3(kThreads), 0, st, a);
@@ -1035,9 +1050,9 @@ extern "C" int nl_flash_attention_bwd(void* stream, int batch, int heads, int se
   NL_TRY(fill_bwd(a, seq, causal, scale, Q, sq, K, sk, V, sv, dO, sdo, L, D));
   NL_TRY(check_op(dQ, sdq, "dQ"));
   a.dq = OutOp{dQ, sdq};
+  const int ks = bwd_groups(batch, heads, seq);
   dim3 grid;
-  int ks;
-  NL_TRY(tile_grid(batch, heads, seq, grid, ks));
+  NL_TRY(tile_grid(batch, heads, seq, ks, grid));  // refused before anything is launched
   // With two wave groups dQ goes first and forms D on the way, which dK/dV then
   // reads: the preprocess launch (4 us) is a tenth of such a backward. On a full
   // chip D's O rows would only lengthen the start of every dQ workgroup: at 32 x
