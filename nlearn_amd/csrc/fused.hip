@@ -12,8 +12,8 @@
 //         dgamma = sum_rows dy * xh,  dbeta = sum_rows dy
 //
 // MI355X design: one 64-lane wave per row (a 512-wide bf16 row is one 16-byte
-// vector per lane), wavefront butterflies for the row statistics, no LDS in
-// the forward. Parameter-gradient sums are per-workgroup partial rows combined
+// vector per lane), wave sums by DPP adds and row swaps for the row statistics,
+// no LDS in the forward. Parameter-gradient sums are per-workgroup partial rows combined
 // in a fixed order by a second kernel (deterministic, no atomics).
 #include <type_traits>
 
@@ -24,7 +24,7 @@ namespace {
 
 constexpr int kRowsPerBlock = 4;   // LayerNorm: one wave per row, 4 waves per workgroup
 constexpr int kMaxD = 4096;        // LayerNorm width limit (8 vectors of 8 per lane)
-constexpr int kLnBwdBlocks = 1024; // LayerNorm backward: partial rows of dgamma / dbeta the workspace holds
+constexpr int kLnBwdBlocks = 1024; // LayerNorm backward: most workgroups, and the partial rows of dgamma / dbeta the workspace holds
 constexpr int kColsumRows = 64;    // column sums: rows per partial
 
 // Lane `lane` holds columns (i*64 + lane)*8 .. +7 of the row in vector i.
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void ln_fwd_kernel(int rows, in
 // columns [4q, 4q+4) of its strip; the 64 phase sums are then added in groups
 // of 4 (phases 4g..4g+3) and the 16 group sums in g order. The strips are
 // narrow so that a 512-column sum still spreads over 32 workgroups per pair
-// with every row load in flight at once (P <= 512: 8 loads a thread).
+// with every row load in flight at once (LayerNorm's P <= 1024: 16 loads a thread).
 __device__ __forceinline__ void sum_partials_strip(int bx, int pair, int P, int D, const float* __restrict__ part0,
                                                    float* __restrict__ out0, const float* __restrict__ part1,
                                                    float* __restrict__ out1, int accumulate) {
@@ -711,8 +711,16 @@ int vectors_per_lane(int D) {
 // to keep the loads in flight. Measured with the sum (us, 1024 / 512 / 256):
 //   4096 x 512   15.1 / 11.6 / 10.3     16384 x 512   24.0 / 21.3 / 26.1
 //   8192 x 512   18.4 / 14.7 / 16.0     32768 x 512   35.9 / 32.2 / 43.0
-int ln_bwd_blocks(int rows) {
-  return std::min(rows >= 8192 ? 512 : 256, (rows + kRowsPerBlock - 1) / kRowsPerBlock);
+//   8191 x 1024  25.2 / 19.4 / 19.6     8191 x 2048   47.0 / 36.5 / 31.5
+// A row of up to 256 columns leaves half of a wave's lanes or more without a
+// load, so the same bytes need more waves, most of all where the sum is left to
+// the next call (us of nl_layernorm_bwd_deferred, 1024 / 768 / 512 / 256):
+//   4096 x 256    5.1 /  4.8 /  4.4 /  5.1    32768 x 256  17.3 / 17.4 / 18.8 / 27.7
+//   8191 x 256    6.3 /  5.7 /  6.0 /  7.6    65536 x 256  28.1 / 28.9 / 32.2 / 51.1
+int ln_bwd_blocks(int rows, int D) {
+  const int most = D > 256 ? (rows >= 8192 ? 512 : 256)
+                           : (rows >= 49152 ? kLnBwdBlocks : rows >= 20000 ? 768 : rows >= 5000 ? 512 : 256);
+  return std::min(most, (rows + kRowsPerBlock - 1) / kRowsPerBlock);
 }
 
 }  // namespace
@@ -774,7 +782,7 @@ int ln_bwd_launch(void* stream, int rows, int D, const nl_bf16* dy, const nl_bf1
                   const PartialSums& prev, const char* who) {
   if (rows < 0 || D <= 0 || (D % 8) != 0 || D > kMaxD)
     return nl_set_error(NL_EINVAL, std::string(who) + ": need 0 < D <= 4096 and D % 8 == 0");
-  const int nblk = rows > 0 ? ln_bwd_blocks(rows) : 0;
+  const int nblk = rows > 0 ? ln_bwd_blocks(rows, D) : 0;
   if (rows > 0) {
     if (!dy || !x || !mean || !rstd || !gamma || !dx || !ws)
       return nl_set_error(NL_EINVAL, std::string(who) + ": null pointer");
@@ -812,7 +820,7 @@ int partial_sums_of(int rows, int D, const void* ws, float* dgamma, float* dbeta
     return nl_set_error(NL_EINVAL, std::string(who) + ": partial sums need 0 < D <= 4096 and D % 8 == 0");
   if (!dgamma || !dbeta) return nl_set_error(NL_EINVAL, std::string(who) + ": null dgamma or dbeta");
   if (((uintptr_t)ws & 15) != 0) return nl_set_error(NL_EALIGN, std::string(who) + ": partials must be 16-byte aligned");
-  out.P = ln_bwd_blocks(rows);
+  out.P = ln_bwd_blocks(rows, D);
   out.D = D;
   out.strips = (D + 15) / 16;
   out.part_g = static_cast<const float*>(ws);
@@ -834,7 +842,7 @@ extern "C" int nl_layernorm_bwd(void* stream, int rows, int D, const nl_bf16* dy
   if (!dgamma || !dbeta) return nl_set_error(NL_EINVAL, "layernorm_bwd: null pointer");
   NL_TRY(ln_bwd_launch(stream, rows, D, dy, x, mean, rstd, gamma, dres, dx, ws, ws_bytes, no_partial_sums(),
                        "layernorm_bwd"));
-  const int blocks = ln_bwd_blocks(rows);
+  const int blocks = ln_bwd_blocks(rows, D);
   const float* pg = static_cast<const float*>(ws);
   hipLaunchKernelGGL(sum_partials_kernel, dim3((D + 15) / 16, 2), dim3(256), 0, (hipStream_t)stream, blocks, D, pg,
                      dgamma, pg + (size_t)blocks * D, dbeta, accumulate);

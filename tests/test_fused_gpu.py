@@ -86,10 +86,14 @@ def test_layernorm_fwd_bwd(dev, rows, D, residual):
         assert torch.equal(a, c)                           # fixed reduction order
 
 
-@pytest.mark.parametrize("rows,D", [(1023, 512), (1026, 512), (8191, 256), (8193, 264)])
+@pytest.mark.parametrize("rows,D", [(1023, 512), (1026, 512), (8191, 256), (8193, 264),
+                                    (4999, 64), (5001, 256), (20003, 128), (49155, 64),   # narrow rows: 256 / 512 / 768 / 1024
+                                    (2051, 1024), (1500, 2048), (1030, 4096)])            # several vectors per lane
 def test_layernorm_around_the_workgroup_limits(dev, rows, D):
-    """Row counts around the backward's two workgroup limits (256 up to 8191
-    rows, 512 above), where waves take unequal numbers of rows."""
+    """Row counts around the backward's workgroup limits (256 up to 8191 rows, 512
+    above; rows of up to 256 columns 256, 512, 768, 1024 from 5000, 20000, 49152
+    rows), where waves take unequal numbers of rows, and rows of several vectors
+    per lane over waves that take more than one."""
     test_layernorm_fwd_bwd(dev, rows, D, True)
 
 
