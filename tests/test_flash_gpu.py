@@ -83,10 +83,14 @@ def test_flash_ragged_sequences(dev, B, H, S, causal):
     _check_against_oracle((O, L, dq, dk, dv), f32, B, H, S, causal)
 
 
-@pytest.mark.parametrize("B,H,S", [(2, 128, 33), (257, 1, 65), (52, 5, 97), (43, 3, 257)])
+@pytest.mark.parametrize("B,H,S", [(2, 128, 33), (257, 1, 65), (52, 5, 97), (43, 3, 257),
+                                   # two groups with blocks for both, uneven and in several query tiles
+                                   (2, 8, 777), (1, 3, 257), (2, 3, 130),
+                                   # the forward's own lines: 64 rows, and two workgroups per CU
+                                   (2, 3, 64), (8, 8, 255), (8, 8, 256), (4, 8, 767), (4, 8, 768)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_flash_tile_counts_on_both_sides(dev, B, H, S, causal):
-    """Ragged sequences at 256 tiles of 128 rows (two wave groups per
+    """Ragged sequences at up to 256 tiles of 128 rows (two wave groups per
     workgroup) and just above (one), and the backward's parts against the
     whole: D formed inside the dQ kernel, dQ, dK and dV equal those of the
     preprocess, dK/dV and dQ entry points bit for bit."""
@@ -132,7 +136,7 @@ def test_flash_bwd_over_an_input(dev, B, H, S, out, over):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("B,H,S", [(1, 2, 545), (2, 1, 1024)])
+@pytest.mark.parametrize("B,H,S", [(1, 2, 545), (2, 1, 1024), (65, 1, 545)])   # two wave groups; one (325 tiles)
 @pytest.mark.parametrize("causal", [True, False])
 def test_flash_scores_growing_along_the_keys(dev, B, H, S, causal):
     """Scores that grow along the keys by about 45 log2 units over the
@@ -246,13 +250,14 @@ def test_flash_reference_api_autograd(dev):
     assert rel_l2(_np(V.grad), rdv) <= TOL
 
 
-def test_flash_never_reads_beyond_causal_blocks(dev):
+@pytest.mark.parametrize("B,H", [(1, 2), (130, 1)])   # two wave groups per workgroup; one (260 tiles)
+def test_flash_never_reads_beyond_causal_blocks(dev, B, H):
     """Keys/values at positions >= 128 are poisoned with NaN: the first 128
     queries' outputs (and the dQ of those queries) must be unchanged."""
     import torch
     from nlearn_amd.attention import flash_bwd_raw4, flash_fwd_raw4
 
-    (q, k, v, do), _ = _rand_case(dev, 1, 2, 256, seed=77)
+    (q, k, v, do), _ = _rand_case(dev, B, H, 256, seed=77)
     O1, L1 = flash_fwd_raw4(q, k, v)
     dq1, _, _ = flash_bwd_raw4(q, k, v, O1, do, L1)
     k2, v2 = k.clone(), v.clone()

@@ -251,15 +251,18 @@ def test_gemm_tall_tile_path_exact_small_integers(dev, opA, M, N, K):
 @pytest.mark.parametrize("M,N,K", [
     (63, 65, 128), (64, 64, 127), (129, 190, 257), (4096, 512, 130),   # 64 x 64 tiles (the last: as many as they take)
     (70, 66, 2049), (130, 200, 5000),                                  # ... split over K
-    (2000, 1100, 192), (8130, 500, 65), (2048, 2047, 64),              # 128 x 64 tiles
+    (70, 66, 8200),                                                    # ... of the fewest tiles, past K = 4096
+    (2000, 1100, 192), (8130, 500, 65), (2048, 2047, 64),              # 128 x 64 tiles (some epilogues and forms)
+    (1100, 2000, 1088), (2047, 1030, 768), (500, 8100, 1000),          # ... with more of K, and at its edge
+    (70, 200, 64), (2050, 500, 192), (4090, 500, 448),                 # K = 64 past whole 128-k stages
     (2100, 2100, 200)])                                                # 128 x 128 tiles, one pass
 def test_gemm_small_product_tiles(dev, opA, opB, M, N, K):
     """Tile edges and K remainders of the tiles for products that do not fill
     the chip, and of the next larger ones: fp32 and bf16 outputs, beta, and the
-    bias / GELU' epilogues (after the reduction where K is split). Small
-    integers: products and sums are exact in fp32."""
+    bias, bias + GELU and GELU' epilogues (after the reduction where K is split).
+    Small integers: products and sums are exact in fp32."""
     import torch
-    from nlearn_amd.kernels.gemm import EPI_BIAS, EPI_DGELU, gemm_raw, padded_empty
+    from nlearn_amd.kernels.gemm import EPI_BIAS, EPI_BIAS_GELU, EPI_DGELU, gemm_raw, padded_empty
     from oracle import model_np as om
 
     rng = np.random.default_rng(M + 7 * N + 13 * K)
@@ -278,6 +281,9 @@ def test_gemm_small_product_tiles(dev, opA, opB, M, N, K):
     gemm_raw(Ad, Bd, opA, opB, out=c0, beta=2.0)
     eb = gemm_raw(Ad, Bd, opA, opB, out_dtype=torch.bfloat16, epi=EPI_BIAS, bias=torch.from_numpy(bias).to(dev))
     ed = gemm_raw(Ad, Bd, opA, opB, alpha=0.25, epi=EPI_DGELU, aux=ud)
+    pre = padded_empty(M, N, torch.bfloat16, dev)
+    eg = gemm_raw(Ad, Bd, opA, opB, out_dtype=torch.bfloat16, alpha=0.125, epi=EPI_BIAS_GELU,
+                  bias=torch.from_numpy(bias).to(dev), aux=pre)
     torch.cuda.synchronize()
     assert np.array_equal(_np(f), ref)
     assert np.array_equal(_np(b), ops.bf16_round(ref))
@@ -285,6 +291,9 @@ def test_gemm_small_product_tiles(dev, opA, opB, M, N, K):
     assert np.array_equal(_np(eb), ops.bf16_round(ref + bias))
     _, t = om._gelu(u.astype(np.float64))
     assert rel_l2(_np(ed), om._gelu_bwd(0.25 * ref, u.astype(np.float64), t)) <= 1e-5   # as the epilogue test's bound
+    # eighths: exact in fp32, one rounding to the saved bf16; gelu of that within one more
+    assert np.array_equal(_np(pre), ops.bf16_round(0.125 * ref + bias))
+    assert rel_l2(_np(eg), om._gelu(_np(pre).astype(np.float64))[0]) <= 4e-3
 
 
 @pytest.mark.parametrize("M,N,K", [(512, 512, 2048), (512, 1536, 4096), (300, 1000, 1900), (2000, 1100, 4096)])
