@@ -28,10 +28,10 @@
 //     loads are in flight while the current one is consumed.
 //   * Causal work skipping per wave; fully masked waves only join the barriers.
 //     The heaviest tiles are launched first.
-//   * Few tiles (tile_grid): two wave groups per workgroup, 64 rows, each group
-//     every other block of the streamed side with buffers of its own; their
-//     partial results are combined in LDS. What bounds such a call is the chain
-//     of blocks of its longest tile on a chip that is not full.
+//   * Few tiles (fwd_groups, bwd_groups): two wave groups per workgroup, 64 rows,
+//     each group every other block of the streamed side with buffers of its own;
+//     their partial results are combined in LDS. What bounds such a call is the
+//     chain of blocks of its longest tile on a chip that is not full.
 #include <type_traits>
 #include <algorithm>
 #include <atomic>

@@ -26,7 +26,7 @@
 //   * Products too small to fill the chip (a few thousand tokens) take 64 x 64
 //     tiles with 128-k stages, or 128 x 64 ones: they wait on the DMA round trip
 //     of each stage, so more, smaller workgroups and fewer stages are what
-//     helps. make_plan draws the lines, with the times on both sides.
+//     helps. small_plan draws the lines, with the times on both sides.
 //   * 256 x 256 tiles (8 waves, the LM head) bound by the CU's global -> LDS
 //     path; in the weight-gradient (TN) form half of the waves issue each
 //     stage's DMA, so one wave per SIMD computes while the other queues loads.
@@ -1289,9 +1289,9 @@ int cu_count() {
 
 enum Tile { kTile64, kTile128x64, kTile128, kTile256x128, kTile256 };
 
-// Tile configuration and K split of one product (shared by the workspace query:
-// the split depends on neither the epilogue nor the output type where it is below
-// the 256 x 256 tiles' line).
+// Tile configuration and K split of one product, shared by the workspace query.
+// That knows neither epilogue nor output type: small products split by their
+// sizes alone, and a call whose plan needs more than it was given runs unsplit.
 struct Plan {
   Tile tile;
   int tiles;

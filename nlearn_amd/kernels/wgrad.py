@@ -61,8 +61,7 @@ def overlap_weight_grads(device=None):
     if _active is not None:
         raise RuntimeError("overlap_weight_grads() does not nest")
     dev = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
-    _active = {"side": _side_stream(dev), "keep": [], "main": torch.cuda.current_stream(dev), "forked": False,
-               "dev": dev}
+    _active = {"side": _side_stream(dev), "keep": [], "main": torch.cuda.current_stream(dev), "forked": False}
     try:
         yield
     finally:
