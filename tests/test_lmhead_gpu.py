@@ -1,6 +1,7 @@
 """The LM head + cross-entropy with the CE of each row chunk pipelined behind
 the next chunk's logits GEMM (kernels.cross_entropy.lm_head_cross_entropy)
-must equal the unchunked linear + cross_entropy bit for bit: loss, dX and dW."""
+must equal the unchunked linear + cross_entropy bit for bit up to d = 1024: loss,
+dX and dW."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,9 @@ pytestmark = pytest.mark.gpu
                                             (16384, 512, 50257, 2, 2.0), (3000, 512, 50257, 2, 1.0),
                                             # the whole and its chunks on different tiles, K above 512 or ragged
                                             (600, 320, 4096, 2, 1.0), (1024, 768, 8192, 2, 1.0),
-                                            (513, 1000, 4100, 2, 1.0), (1024, 1024, 4104, 2, 1.0)])
+                                            (513, 1000, 4100, 2, 1.0), (1024, 1024, 4104, 2, 1.0),
+                                            # ... the whole on 256 x 256 ones, persistent and with a K tail
+                                            (4096, 1024, 16400, 2, 1.0), (4096, 1000, 16400, 2, 1.0)])
 def test_lm_head_cross_entropy_equals_linear_then_ce(dev, M, d, V, chunks, g):
     import torch
     from nlearn_amd.kernels.cross_entropy import cross_entropy, lm_head_cross_entropy
